@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
+#include <utility>
 
 #include "prefill_mfma.h"
 
@@ -13,6 +14,7 @@ namespace {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 // Native vector for staged K/V rows (HIP's uint4 struct is copied with memcpy,
 // which keeps the staging registers in scratch memory).
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -24,6 +26,10 @@ template <> struct Mfma<_Float16> {
     __device__ static inline f32x4 mma(const uint4& a, const uint4& b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    }
+    __device__ static inline f32x16 mma32(const uint4& a, const uint4& b, f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
     __device__ static inline uint32_t pack2(float x, float y) { return pack_h2(x, y); }
     static constexpr uint32_t kOnes = 0x3C003C00u;   // two halves of 1.0
@@ -778,23 +784,19 @@ void prefill_mfma_kernel(MfmaPrefillArgs a) {
 //                 (keys 4g .. 4g + 3 of one dim) per four k-steps.
 // Softmax row sums are kept per lane (its own keys) and reduced over the four
 // lanes of a query column at the end.
-// LDS tile buffers and occupancy.  head_dim 64: K double-buffered, V^T
-// single (53 KB), three waves per SIMD (the compiler spills ~60 registers to
-// reach 168; still 13 % faster than two waves without spills).  head_dim 128:
-// ~300 registers, one wave per SIMD, so both tiles double-buffered (137 KB).
-// The S = K Q^T cluster at raised wave priority (as in the 16-bit kernel):
-// configuration 4's shape in fp32 360-380 -> 339-344 us; neutral at
-// head_dim 128 (one wave per SIMD).
+// Instantiated for head_dim 256 alone: the smaller head dims run faster on
+// prefill_f32_split_kernel, whose two tiles of two planes would take 128 KB of
+// LDS here and its operands more registers than a wave has.  One work-group per
+// CU, single-buffered tiles (134 KB).
+// The S = K Q^T cluster runs at raised wave priority (as in the 16-bit kernel).
 template <int D>
 struct SmemF32 {
-    static constexpr int KNB = D == 64 || D == 128 ? 2 : 1;
-    static constexpr int VNB = D == 128 ? 2 : 1;   // 64, 96, 256: 1
     static constexpr int KPAD = D + 4;    // floats per K row (pad: 16-byte reads of 16 rows hit distinct banks)
     static constexpr int VPAD = BN + 4;   // floats per V^T row
     union {
         struct {
-            alignas(16) float k[KNB][BN * KPAD];
-            alignas(16) float vt[VNB][D * VPAD];
+            alignas(16) float k[BN * KPAD];
+            alignas(16) float vt[D * VPAD];
         };
         int order[6 * kRankUnits];
     };
@@ -802,15 +804,15 @@ struct SmemF32 {
 };
 
 template <int D, bool CG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : (D == 96 ? 2 : 1))))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
 void prefill_f32_kernel(MfmaPrefillArgs a) {
     typedef SmemF32<D> S;
-    constexpr int KPAD = S::KPAD, VPAD = S::VPAD, KNB = S::KNB, VNB = S::VNB;
+    constexpr int KPAD = S::KPAD, VPAD = S::VPAD;
     constexpr int KB = D / 16;              // 16-dim blocks of the QK^T product
     constexpr int DT = D / 16;              // 16-dim tiles of the output
     constexpr int KCH_T = BN * D / 4 / 256;          // 16-byte K chunks per thread
     constexpr int VT_N = (BN / 4) * (D / 4);           // V tasks (4 keys x 4 dims) per tile
-    constexpr int VT_T = (VT_N + 255) / 256;           // per thread (head_dim 96: the last partly idle)
+    constexpr int VT_T = (VT_N + 255) / 256;           // per thread
     __shared__ S sm;
 
     const int tid = threadIdx.x;
@@ -921,15 +923,15 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
             for (int r = 0; r < 4; ++r) vr[j][r] = *reinterpret_cast<const u32x4*>(p + r * row_bytes);
         }
     };
-    auto store_k = [&](int buf) {
+    auto store_k = [&]() {
 #pragma unroll
         for (int j = 0; j < KCH_T; ++j) {
             const int ch = tid + 256 * j;
             const int key = ch / (D / 4), c = ch % (D / 4);
-            *reinterpret_cast<u32x4*>(&sm.k[buf][key * KPAD + c * 4]) = kr[j];
+            *reinterpret_cast<u32x4*>(&sm.k[key * KPAD + c * 4]) = kr[j];
         }
     };
-    auto store_v = [&](int buf) {
+    auto store_v = [&]() {
 #pragma unroll
         for (int j = 0; j < VT_T; ++j) {
             const int task = tid + 256 * j;
@@ -937,7 +939,7 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
             const int kq = task % (BN / 4), c = task / (BN / 4);
 #pragma unroll
             for (int e = 0; e < 4; ++e)   // 4x4 transpose: V^T row 4c + e, keys 4kq .. 4kq+3
-                *reinterpret_cast<u32x4*>(&sm.vt[buf][(4 * c + e) * VPAD + 4 * kq]) =
+                *reinterpret_cast<u32x4*>(&sm.vt[(4 * c + e) * VPAD + 4 * kq]) =
                     u32x4{vr[j][0][e], vr[j][1][e], vr[j][2][e], vr[j][3][e]};
         }
     };
@@ -952,14 +954,12 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
         load_q();
         load_k(t_begin);
         load_v(t_begin);
-        store_k(0);
-        store_v(0);
+        store_k();
+        store_v();
     }
     __syncthreads();
 
     for (int t = t_begin; t < t_end; ++t) {
-        const int kbuf = KNB == 2 ? (t - t_begin) & 1 : 0;
-        const int vbuf = VNB == 2 ? (t - t_begin) & 1 : 0;
         const bool next = t + 1 < t_end;   // uniform
         if (next) {
             if (4 * (t + 1) + 4 > tbase + kPageWindow) stage_pages(4 * (t + 1));
@@ -984,7 +984,7 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb) {
                 const float4 ka = *reinterpret_cast<const float4*>(
-                    &sm.k[kbuf][(16 * kt + c16) * KPAD + kb * 16 + g * 4]);
+                    &sm.k[(16 * kt + c16) * KPAD + kb * 16 + g * 4]);
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) {
                     f32x4& acc = kb < KB / 2 ? s[kt][nt] : hi[nt];
@@ -999,8 +999,8 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
         }
         LLKV_PF_PRIO(true, 0);
         if (next) {
-            if (KNB == 1) __syncthreads();   // every wave is done with the K buffer
-            store_k(KNB == 2 ? kbuf ^ 1 : 0);
+            __syncthreads();   // every wave is done with the K buffer
+            store_k();
             load_v(t + 1);
         }
 
@@ -1061,7 +1061,7 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
                 const float4 va = *reinterpret_cast<const float4*>(
-                    &sm.vt[vbuf][(dt * 16 + c16) * VPAD + 16 * kt + 4 * g]);
+                    &sm.vt[(dt * 16 + c16) * VPAD + 16 * kt + 4 * g]);
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) {
                     o[dt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(va.x, s[kt][nt][0], o[dt][nt], 0, 0, 0);
@@ -1073,8 +1073,8 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
         }
 
         if (next) {
-            if (VNB == 1) __syncthreads();   // every wave is done with the V^T buffer
-            store_v(VNB == 2 ? vbuf ^ 1 : 0);
+            __syncthreads();   // every wave is done with the V^T buffer
+            store_v();
         }
         __syncthreads();
     }
@@ -1098,6 +1098,543 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
                 make_float4(o[dt][nt][0] * inv, o[dt][nt][1] * inv, o[dt][nt][2] * inv, o[dt][nt][3] * inv);
         if (!wk.direct && g == 0) a.part_lse[pidx * BQ + row] = lt > 0.f ? m[nt] + fast_log2(lt) : -INFINITY;
     }
+}
+
+// fp32 pools at head_dim 64 / 96 / 128: both products on the fp16 matrix
+// instructions, every operand, scaled by a power of two, as the sum of two fp16
+// terms x = x1 + x2 (x1 = fp16(x), x2 = fp16(x - x1)), and three of the four
+// partial products,
+//     x y = x2 y1 + x1 y2 + x1 y1    (x2 y2 <= 2^-22 |x y| is dropped),
+// summed in fp32.  The fp32 form on v_mfma_f32_16x16x4_f32 ran at 61 % of that
+// instruction's rate (354 us for eight 512-row chunks on prefixes up to 4096,
+// 14/2/64); v_mfma_f32_32x32x16_f16 has 16 times the rate, so the three products
+// cost 0.19 of its matrix time, and the splits are VALU work that runs beside
+// the MFMAs: 158 us there, and 69 -> 37 us for a first prefill of 8 x 77 .. 512
+// rows.  Bound now by the latency of a tile's loads and by VALU issue (two
+// waves per SIMD at 256 registers; one at head_dim 96 / 128).  Three bf16 terms (exact) with six products measured 200 us there:
+// with random data the matrix cores sustain about two thirds of their nominal
+// rate, so the number of products decides.
+//
+// Error.  A term pair holds 22 bits, one or two less than fp32; a score's sum
+// takes 3 D / 16 roundings instead of D / 4 and the output's 12 per 64 keys
+// instead of 16, and those dominate: against 64 bits the result is nearer than
+// the fp32 form's (4.1e-7 there at the shape above).  Below 2^-14 a term is
+// subnormal: with the scales 2^6 (Q, K), 2^8 (V) and 2^7 (P) its rounding is
+// <= 2^-31 absolute, so a tile counts as fit when its largest magnitude is in
+// [2^-8, 2^9] (2^-10, 2^7 for V) or zero, and the rounding is then <= 2^-23 of
+// that magnitude.  A tile or a Q that is not fit (infinities included) runs on
+// the fp32 matrix instructions: it is staged again as plain fp32, high halves in
+// the first plane and low halves in the second.
+//
+// K and V tiles lie in LDS as two planes with the operand layout of the 16-bit
+// kernel (V^T by transposing reads), split once per work-group while staging.
+constexpr float kScaleQK = 64.0f, kScaleV = 256.0f, kShiftP = 7.0f;   // P: 2^7
+constexpr float kFitMax = 32768.0f, kFitMin = 0.25f;                  // scaled magnitudes
+
+// x - float(low / high half of w): one v_fma_mix_f32 each.
+__device__ inline float minus_lo(float x, uint32_t w) {
+    return __builtin_fmaf((float)__builtin_bit_cast(half2_v, w).x, -1.0f, x);
+}
+__device__ inline float minus_hi(float x, uint32_t w) {
+    return __builtin_fmaf((float)__builtin_bit_cast(half2_v, w).y, -1.0f, x);
+}
+
+// The two fp16 terms of 8 values, two per word.
+__device__ inline void split8(const float (&x)[8], uint4 (&t)[2]) {
+    uint32_t w[2][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        w[0][j] = pack_h2(x[2 * j], x[2 * j + 1]);
+        w[1][j] = pack_h2(minus_lo(x[2 * j], w[0][j]), minus_hi(x[2 * j + 1], w[0][j]));
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) t[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+}
+
+// 8 plain fp32 values in the same place, and element e of them.
+__device__ inline void plain8(const float (&x)[8], uint4 (&t)[2]) {
+    uint32_t w[2][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t a = __float_as_uint(x[2 * j]), b = __float_as_uint(x[2 * j + 1]);
+        w[0][j] = (a >> 16) | (b & 0xFFFF0000u);
+        w[1][j] = (a & 0xFFFFu) | (b << 16);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) t[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+}
+__device__ inline float plain(const uint4 (&t)[2], int e) {
+    const uint32_t h = e < 2 ? t[0].x : (e < 4 ? t[0].y : (e < 6 ? t[0].z : t[0].w));
+    const uint32_t l = e < 2 ? t[1].x : (e < 4 ? t[1].y : (e < 6 ? t[1].z : t[1].w));
+    return __uint_as_float((e & 1) ? (h & 0xFFFF0000u) | (l >> 16) : (h << 16) | (l & 0xFFFFu));
+}
+
+// Uniform over the wave: the largest magnitudes `most` of its lanes do not fit
+// the two terms.  (A NaN passes as one: it stays NaN in either form.)
+__device__ inline bool unfit(float most) {
+    return __builtin_amdgcn_ballot_w64(most > kFitMax) != 0 ||
+           (__builtin_amdgcn_ballot_w64(most >= kFitMin) == 0 && __builtin_amdgcn_ballot_w64(most > 0.0f) != 0);
+}
+
+// f(integral_constant 0), ..., f(integral_constant N - 1).
+template <class F, int... I>
+__device__ inline void static_for_impl(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>()), ...);
+}
+template <int N, class F>
+__device__ inline void static_for(F f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>());
+}
+
+// The three products in the order of accumulation: term of A, term of B.
+constexpr int kSplitA[3] = {1, 0, 0};
+constexpr int kSplitB[3] = {0, 1, 0};
+
+// split8 of 2 N values times `scale` in 2 N steps of three VALU instructions or
+// so, to be issued one by one between MFMAs: a 32x32x16 MFMA holds the matrix
+// core for 32 cycles, in which a wave can issue VALU instructions, but only
+// those that stand between it and the next MFMA (issue is in order, and the
+// compiler by itself puts all VALU work of a region on one side of its MFMAs).
+template <int N>
+struct SplitSeq {
+    static constexpr int kSteps = 2 * N;
+    float x[2 * N];
+    uint32_t w[2][N];
+    float most;   // largest scaled magnitude (step 0 starts it)
+    template <bool FIT>
+    __device__ void step(int i, float scale) {
+        const int j = i >> 1;
+        float &a = x[2 * j], &b = x[2 * j + 1];
+        if ((i & 1) == 0) {
+            if constexpr (FIT) {
+                a *= scale;
+                b *= scale;
+                const float ab = fmaxf(fabsf(a), fabsf(b));
+                most = i == 0 ? ab : fmaxf(most, ab);
+            }
+            w[0][j] = pack_h2(a, b);
+        } else {
+            w[1][j] = pack_h2(minus_lo(a, w[0][j]), minus_hi(b, w[0][j]));
+        }
+    }
+    __device__ uint4 term(int p, int c) const {   // values 8 c .. 8 c + 7
+        return make_uint4(w[p][4 * c], w[p][4 * c + 1], w[p][4 * c + 2], w[p][4 * c + 3]);
+    }
+};
+
+template <int D>
+struct SmemSplit {
+    static constexpr bool kSwz = (D & (D - 1)) == 0;      // 16-byte chunks XOR-swizzled by row, else rows padded
+    static constexpr int PAD = kSwz ? D : D + 8;          // halves per row
+    union {
+        struct {
+            alignas(16) uint16_t k[2][BN * PAD];
+            alignas(16) uint16_t v[2][BN * PAD];
+        };
+        int order[6 * kRankUnits];
+    };
+    int pages[kPageWindow];
+    int plain[2][2];   // [K, V][tile parity]: the latest such tile that does not fit two terms
+    int plain_q;       // a wave's Q does not fit
+};
+
+template <int D, bool CG>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1)))
+void prefill_f32_split_kernel(MfmaPrefillArgs a) {
+    typedef SmemSplit<D> S;
+    constexpr int PAD = S::PAD;
+    constexpr int CPR = D / 8;              // 8-value chunks per row
+    constexpr int KS = D / 16;              // k-steps of the QK^T product
+    constexpr int DT = D / 32;              // 32-dim tiles of the output
+    constexpr int CH_T = BN * CPR / 256;    // chunks per thread and tile
+    static_assert(BN * CPR % 256 == 0, "chunks spread evenly over the threads");
+    __shared__ S sm;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, c32 = lane & 31;
+    Work wk;
+    if (!take_work(a, sm.order, wk)) return;
+    if (tid < 5) (&sm.plain[0][0])[tid] = tid < 4 ? -1 : 0;   // (before the barrier of stage_pages / below)
+    // Every wave's reads of its unit from the ranking, which overlays the tile
+    // buffers, complete before any wave writes the first tile (stage_pages has
+    // its own barrier).
+    if constexpr (CG) lds_barrier();
+    poison_uncovered_rows<float, D>(a, wk);
+    const int hq = wk.hq, kvh = wk.kvh, unit = wk.unit, n = wk.n, ci = wk.ci;
+    const int q0 = wk.q0, P = wk.P, q_lo = wk.q_lo, L = wk.L, kend = wk.kend;
+    const int t_begin = wk.t_begin, t_end = wk.t_end;
+    const int last_page = L > 0 ? (L - 1) / kPage : 0;
+    const int* bt = a.bt + (int64_t)n * a.max_blocks;
+
+    // Q^T operands: lane (h, c32) holds dims 16 ks + 8 h .. + 7 of query c32.
+    const int ql = q_lo + w * WQ + c32;
+    uint4 qop[KS][2];
+    const float* qrow = reinterpret_cast<const float*>(a.q) + ((int64_t)(q0 + ql) * a.Hq + hq) * D + h * 8;
+    auto read_q = [&](int ks, float (&x)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = 0.0f;
+        if (ql < P) {
+            const float4* p = reinterpret_cast<const float4*>(qrow + ks * 16);
+            const float4 lo = p[0], hi = p[1];
+            x[0] = lo.x, x[1] = lo.y, x[2] = lo.z, x[3] = lo.w;
+            x[4] = hi.x, x[5] = hi.y, x[6] = hi.z, x[7] = hi.w;
+        }
+    };
+    auto load_q = [&]() {
+        float most = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            float x[8];
+            read_q(ks, x);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                x[e] *= kScaleQK;
+                most = fmaxf(most, fabsf(x[e]));
+            }
+            split8(x, qop[ks]);
+        }
+        if (unfit(most) && lane == 0) sm.plain_q = 1;
+    };
+    const int qpos = ql < P ? (a.causal ? wk.hist + ql : L - 1) : -1;
+    const int wq0 = q_lo + w * WQ;
+    const int wave_min_pos = (wq0 + WQ <= P) ? (a.causal ? wk.hist + wq0 : L - 1) : -1;
+
+    f32x16 o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
+    float m = kNegBig;
+    float lsum = 0.0f;   // this lane's keys only
+
+    // ---- staging: 8 consecutive values per chunk, global -> registers ->
+    // three planes in LDS ----------------------------------------------------
+    int tbase = 0;
+    const uint32_t row_bytes = (uint32_t)(a.Hkv * D * sizeof(float));
+    const uint32_t page_bytes = row_bytes * kPage;
+    const int64_t kv0 = (int64_t)kvh * D + (CG ? (int64_t)wk.kvo : 0);
+    const char* kb_ = reinterpret_cast<const char*>(reinterpret_cast<const float*>(a.k) + kv0);
+    const char* vb_ = reinterpret_cast<const char*>(reinterpret_cast<const float*>(a.v) + kv0);
+    uint32_t off[CH_T];   // bytes inside the page (paged) / the row (contiguous)
+    int slot[CH_T];       // page of the tile / key of the tile
+    int kdst[CH_T], vdst[CH_T];   // halves inside a plane
+    // Half-column hc of tile row `row` in the K / V planes (swizzled: the 16-byte
+    // chunk index XORed with a permutation of the row's low bits).  K: the 16
+    // lanes of a read phase hold rows 0 .. 15 of one chunk, lanes 0 .. 7 rows
+    // 0 .. 3 and 8 .. 11.  V: a transposing read takes 2 chunks of 4 rows.
+    auto kcol = [&](int row, int hc) {
+        const int b0 = row & 1, b1 = (row >> 1) & 1, b2 = (row >> 2) & 1, b3 = (row >> 3) & 1;
+        if constexpr (D == 64) return (((hc >> 3) ^ (b1 | (b3 << 1) | ((b0 ^ b2) << 2))) << 3) | (hc & 7);
+        if constexpr (D == 128) return (((hc >> 3) ^ (b0 | (b1 << 1) | (b3 << 2) | (b2 << 3))) << 3) | (hc & 7);
+        return hc;
+    };
+    auto vcol = [&](int row, int hc) {
+        const int b0 = row & 1, b1 = (row >> 1) & 1, b2 = (row >> 2) & 1;
+        if constexpr (D == 64) return (((hc >> 3) ^ ((b0 << 1) | (b1 << 2))) << 3) | (hc & 7);
+        if constexpr (D == 128) return (((hc >> 3) ^ ((b2 << 1) | (b0 << 2) | (b1 << 3))) << 3) | (hc & 7);
+        return hc;
+    };
+#pragma unroll
+    for (int j = 0; j < CH_T; ++j) {
+        const int ch = tid + 256 * j;
+        const int key = ch / CPR, c = ch % CPR;
+        slot[j] = CG ? key : key >> 4;
+        off[j] = (CG ? 0u : (uint32_t)(key & 15) * row_bytes) + (uint32_t)c * 32u;
+        kdst[j] = key * PAD + kcol(key, c * 8);
+        vdst[j] = key * PAD + vcol(key, c * 8);
+    }
+    float kraw[CH_T][8], vraw[CH_T][8];
+    auto load_tile = [&](const char* base, int t, float (&raw)[CH_T][8]) {
+        const int* pg = sm.pages + (4 * t - tbase);
+#pragma unroll
+        for (int j = 0; j < CH_T; ++j) {
+            uint64_t at;
+            if constexpr (CG) at = (uint64_t)min(t * BN + slot[j], L - 1) * row_bytes;   // past the last: the last
+            else at = (uint64_t)(uint32_t)max(pg[slot[j]], 0) * page_bytes;
+            const f32x4* p = reinterpret_cast<const f32x4*>(base + at + off[j]);
+            const f32x4 lo = p[0], hi = p[1];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) raw[j][e] = lo[e], raw[j][4 + e] = hi[e];
+        }
+    };
+    // Splits a staged tile into its planes; returns the lane's largest scaled magnitude.
+    auto split_tile = [&](float (&raw)[CH_T][8], uint16_t (&planes)[2][BN * PAD], const int (&dst)[CH_T],
+                          float scale) {
+        float most = 0.0f;
+#pragma unroll
+        for (int j = 0; j < CH_T; ++j) {
+            uint4 tm[2];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                raw[j][e] *= scale;
+                most = fmaxf(most, fabsf(raw[j][e]));
+            }
+            split8(raw[j], tm);
+#pragma unroll
+            for (int p = 0; p < 2; ++p) *reinterpret_cast<uint4*>(&planes[p][dst[j]]) = tm[p];
+        }
+        return most;
+    };
+    // After a split that found tile t of K (kv 0) or V (kv 1) unfit: the whole
+    // tile once more, plain.  Called by every wave (it ends with a barrier).
+    auto restage_plain = [&](uint16_t (&planes)[2][BN * PAD], const int (&dst)[CH_T], const char* base, int t) {
+        float raw[CH_T][8];
+        load_tile(base, t, raw);
+#pragma unroll
+        for (int j = 0; j < CH_T; ++j) {
+            uint4 tm[2];
+            plain8(raw[j], tm);
+#pragma unroll
+            for (int p = 0; p < 2; ++p) *reinterpret_cast<uint4*>(&planes[p][dst[j]]) = tm[p];
+        }
+        lds_barrier();
+    };
+    auto stage_pages = [&](int base) {
+        if constexpr (CG) return;   // no page table
+        tbase = base;
+        for (int i = tid; i < kPageWindow; i += 256) sm.pages[i] = bt[min(base + i, last_page)];
+        lds_barrier();
+    };
+    // A operand of S^T: row c32 of key tile kt holds key 32 kt + (c32 with bits
+    // 2 and 3 exchanged), which makes the 8 scores of each 16-key step that a
+    // lane receives (accumulator rows 8 (i / 4) + 4 h + i % 4) keys 8 h .. 8 h + 7.
+    const int krow = (c32 & 0x13) | ((c32 & 4) << 1) | ((c32 & 8) >> 1);
+    auto k_operand = [&](int kt, int ks, int p) {
+        const int row = 32 * kt + krow;
+        return *reinterpret_cast<const uint4*>(&sm.k[p][row * PAD + kcol(row, ks * 16 + h * 8)]);
+    };
+    // A operand of O^T: lane holds dim 32 dt + c32 of keys 16 j + 8 h .. + 7
+    // (transposing reads, as in the 16-bit kernel).
+    auto v_operand = [&](int dt, int j, uint4 (&va)[2]) {
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        typedef unsigned u32x2v __attribute__((ext_vector_type(2)));
+        const int r0 = 16 * j + 8 * h + ((lane & 15) >> 2), hc = dt * 32 + (lane & 16) + 4 * (lane & 3);
+        const int a0 = r0 * PAD + vcol(r0, hc), a1 = (r0 + 4) * PAD + vcol(r0 + 4, hc);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const u32x2v lo = __builtin_bit_cast(u32x2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4*)(&sm.v[p][a0])));
+            const u32x2v hi = __builtin_bit_cast(u32x2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4*)(&sm.v[p][a1])));
+            va[p] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        }
+    };
+    if (t_begin < t_end) {
+        stage_pages(4 * t_begin);
+        load_tile(kb_, t_begin, kraw);
+        load_tile(vb_, t_begin, vraw);
+        load_q();
+        if (unfit(split_tile(kraw, sm.k, kdst, kScaleQK)) && lane == 0) sm.plain[0][t_begin & 1] = t_begin;
+    }
+    lds_barrier();
+
+    // A tile: QK^T (V of the tile split beside it, its buffer being free since
+    // the last barrier), barrier, softmax and PV (K of the next tile split
+    // beside them), barrier.  The raw values are loaded a phase ahead; the
+    // barriers do not wait for them.
+    for (int t = t_begin; t < t_end; ++t) {
+        const bool next = t + 1 < t_end;   // uniform
+        if (next) {
+            if (4 * (t + 1) + 4 > tbase + kPageWindow) stage_pages(4 * t);   // (tile t: restage_plain)
+            load_tile(kb_, t + 1, kraw);
+        }
+        // (the same for every wave: set before the last barrier)
+        const bool k_plain = __builtin_amdgcn_readfirstlane(sm.plain_q) != 0 ||
+                             __builtin_amdgcn_readfirstlane(sm.plain[0][t & 1]) == t;
+        __builtin_amdgcn_sched_barrier(0);
+
+        // ---- S^T = K Q^T; the lane's scores are keys 32 kt + 16 (i / 8) + 8 h + i % 8
+        f32x16 s[2];
+        float v_most, k_most;
+        float c = a.scale_log2;
+        if (__builtin_expect(!k_plain, 1)) {
+            c *= 1.0f / (kScaleQK * kScaleQK);
+            SplitSeq<4 * CH_T> sq;
+#pragma unroll
+            for (int j = 0; j < CH_T; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sq.x[8 * j + e] = vraw[j][e];
+            uint4 ka[2][2][2];   // [k-step parity][key tile][term]
+            auto read_k = [&](int ks, uint4 (&k2)[2][2]) {
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) k2[kt][p] = k_operand(kt, ks, p);
+            };
+            read_k(0, ka[0]);
+            constexpr int M = 6 * KS, M0 = 4;   // MFMAs; those before V's split (its loads have time to land)
+            static_for<M>([&](auto kc) {
+                constexpr int k = kc, kt = k & 1, ks = k / 6, pr = (k % 6) / 2;
+                if constexpr (k % 6 == 0 && ks + 1 < KS) read_k(ks + 1, ka[(ks + 1) & 1]);
+                s[kt] = Mfma<_Float16>::mma32(ka[ks & 1][kt][kSplitA[pr]], qop[ks][kSplitB[pr]],
+                                              k < 2 ? f32x16{} : s[kt]);
+                if constexpr (k >= M0) {
+                    constexpr int s0 = (k - M0) * sq.kSteps / (M - M0), s1 = (k + 1 - M0) * sq.kSteps / (M - M0);
+                    static_for<s1 - s0>([&](auto ec) {
+                        constexpr int st = s0 + ec;
+                        sq.template step<true>(st, kScaleV);
+                        if constexpr (st % 8 == 7) {
+#pragma unroll
+                            for (int p = 0; p < 2; ++p)
+                                *reinterpret_cast<uint4*>(&sm.v[p][vdst[st / 8]]) = sq.term(p, st / 8);
+                        }
+                    });
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            v_most = sq.most;
+        } else {
+            restage_plain(sm.k, kdst, kb_, t);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) s[kt] = f32x16{};
+            for (int ks = 0; ks < KS; ++ks) {
+                float x[8];
+                read_q(ks, x);
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt) {
+                    const uint4 ka[2] = {k_operand(kt, ks, 0), k_operand(kt, ks, 1)};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)   // contracts dims 16 ks + 8 h + e
+                        s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(plain(ka, e), x[e], s[kt], 0, 0, 0);
+                }
+            }
+            v_most = split_tile(vraw, sm.v, vdst, kScaleV);
+        }
+        if (unfit(v_most) && lane == 0) sm.plain[1][t & 1] = t;
+        lds_barrier();   // V of the tile is in LDS; every wave is done with the K buffer
+        const bool v_plain = __builtin_amdgcn_readfirstlane(sm.plain[1][t & 1]) == t;   // the same for every wave
+        if (__builtin_expect(v_plain, 0)) restage_plain(sm.v, vdst, vb_, t);
+        if (next) load_tile(vb_, t + 1, vraw);
+
+        // ---- mask and online softmax (as the 16-bit kernel) ----------------
+        const int key0 = t * BN;
+        const bool unmasked = key0 + BN - 1 <= wave_min_pos && key0 + BN <= kend;
+        if (!unmasked) {
+            const int r = min(qpos, kend - 1) - key0 - 8 * h;
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (32 * kt + 16 * (i >> 3) + (i & 7) > r) s[kt][i] = -INFINITY;
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[kt][i]);
+        mx *= c;
+        if (__builtin_amdgcn_ballot_w64(mx > m + 8.0f) != 0) {
+            const float mnew = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));
+            const float corr = fast_exp2(m - mnew);
+            m = mnew;
+            lsum *= corr;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] *= corr;
+        }
+
+        // ---- P = 2^(S c - m + 7), O^T += V^T P^T, one 16-key step at a time --
+        const float mp = m - kShiftP;
+        if (__builtin_expect(!v_plain, 1)) {
+            uint4 pop[2];
+            {
+                float p[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    p[e] = fast_exp2(fmaf(s[0][e], c, -mp));
+                    lsum += p[e];
+                }
+                split8(p, pop);
+            }
+            SplitSeq<4 * CH_T> sq;   // the next tile's K (after the last tile: into a buffer nobody reads)
+#pragma unroll
+            for (int j = 0; j < CH_T; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sq.x[8 * j + e] = kraw[j][e];
+            static_for<4>([&](auto jc) {
+                constexpr int j = jc, M = 3 * DT;   // MFMAs of the step
+                uint4 va[DT][2];
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) v_operand(dt, j, va[dt]);
+                SplitSeq<4> ps;   // the next step's probabilities
+                static_for<M>([&](auto kc) {
+                    constexpr int k = kc, dt = k % DT, pr = k / DT;
+                    o[dt] = Mfma<_Float16>::mma32(va[dt][kSplitA[pr]], pop[kSplitB[pr]], o[dt]);
+                    if constexpr (j < 3) {   // 8 exponentials, then their terms
+                        constexpr int s0 = k * 16 / M, s1 = (k + 1) * 16 / M;
+                        static_for<s1 - s0>([&](auto ec) {
+                            constexpr int st = s0 + ec;
+                            if constexpr (st < 8) {
+                                constexpr int e = 8 * (j + 1) + st;
+                                ps.x[st] = fast_exp2(fmaf(s[e >> 4][e & 15], c, -mp));
+                                lsum += ps.x[st];
+                            } else {
+                                ps.template step<false>(st - 8, 1.0f);
+                            }
+                        });
+                    } else {
+                        constexpr int s0 = k * sq.kSteps / M, s1 = (k + 1) * sq.kSteps / M;
+                        static_for<s1 - s0>([&](auto ec) {
+                            constexpr int st = s0 + ec;
+                            sq.template step<true>(st, kScaleQK);
+                            if constexpr (st % 8 == 7) {
+#pragma unroll
+                                for (int p = 0; p < 2; ++p)
+                                    *reinterpret_cast<uint4*>(&sm.k[p][kdst[st / 8]]) = sq.term(p, st / 8);
+                            }
+                        });
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                if constexpr (j < 3) {
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) pop[p] = ps.term(p, 0);
+                }
+            });
+            k_most = sq.most;
+        } else {
+            // (an opaque copy: the exponentials of the two branches must not be
+            // merged and moved ahead of the branch)
+            float mq = mp;
+            asm volatile("" : "+v"(mq));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float p[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    p[e] = fast_exp2(fmaf(s[j >> 1][8 * (j & 1) + e], c, -mq));
+                    lsum += p[e];
+                    p[e] *= kScaleV;   // (V is plain here, scaled in the other tiles)
+                }
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) {
+                    uint4 va[2];
+                    v_operand(dt, j, va);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)   // contracts keys 16 j + 8 h + e
+                        o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(plain(va, e), p[e], o[dt], 0, 0, 0);
+                }
+            }
+            k_most = split_tile(kraw, sm.k, kdst, kScaleQK);
+        }
+        if (unfit(k_most) && lane == 0) sm.plain[0][(t + 1) & 1] = t + 1;
+        lds_barrier();   // K of the next tile is in LDS; every wave is done with the V buffer
+    }
+
+    lsum += __shfl_xor(lsum, 32, 64);
+    if (ql >= P) return;
+    const float inv = lsum > 0.f ? 1.0f / (kScaleV * lsum) : 0.f;
+    const int64_t prow = (((int64_t)unit * a.max_chunks + ci) * a.Hq + hq) * BQ + w * WQ + c32;
+    float* drow = wk.direct ? reinterpret_cast<float*>(a.out) + ((int64_t)(q0 + ql) * a.Hq + hq) * D
+                            : a.part_o + prow * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)   // accumulator rows 8 i + 4 h .. + 3 of dim tile dt
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float4*>(drow + dt * 32 + 8 * i + 4 * h) =
+                make_float4(o[dt][4 * i] * inv, o[dt][4 * i + 1] * inv, o[dt][4 * i + 2] * inv, o[dt][4 * i + 3] * inv);
+    if (!wk.direct && h == 0) a.part_lse[prow] = lsum > 0.f ? m - kShiftP + fast_log2(lsum) : -INFINITY;
 }
 
 // Four consecutive output elements from fp32 values.
@@ -1225,9 +1762,9 @@ PrefillFn kernel16(int head_dim) {
 template <bool CG>
 PrefillFn kernel32(int head_dim) {
     switch (head_dim) {
-        case 64: return prefill_f32_kernel<64, CG>;
-        case 96: return prefill_f32_kernel<96, CG>;
-        case 128: return prefill_f32_kernel<128, CG>;
+        case 64: return prefill_f32_split_kernel<64, CG>;
+        case 96: return prefill_f32_split_kernel<96, CG>;
+        case 128: return prefill_f32_split_kernel<128, CG>;
         default: return prefill_f32_kernel<256, CG>;
     }
 }
