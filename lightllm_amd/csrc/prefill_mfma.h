@@ -56,14 +56,13 @@ struct MfmaPrefillArgs {
     int q_row;
     float scale_log2;
     int qblocks;      // query blocks per sequence
-    int max_chunks;   // key chunks per (sequence, query block)
-    int chunk_tiles;  // key tiles per chunk
-    int groups;       // N * qblocks * max_chunks * Hkv (chunk slot, kv head) work items
-    float* part_o;    // [N*qblocks*max_chunks*Hq][BQ][D] (max_chunks > 1)
-    float* part_lse;  // [N*qblocks*max_chunks*Hq][BQ]
-    // Split decision made on the device from the units' key lengths (max_chunks > 1):
-    // plan_flag (workspace header) receives 1 when the launch runs unsplit after all.
-    int* plan_flag;
+    // Cut key ranges (pick_item): partial slots (0: nothing is cut), launched
+    // items beyond the units, tiles per chunk as a share of the sum of tiles.
+    int max_parts, extra_items;
+    float chunk_share;
+    int2* table;      // per unit: first partial slot, chunks; from the main kernel to the merge
+    float* part_o;    // [max_parts][Hq][BQ][D]
+    float* part_lse;  // [max_parts][Hq][BQ]
     int n_cus;        // compute units of the device
     int resident;     // resident work-groups of the launched kernel
 };

@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <type_traits>
 #include <utility>
@@ -96,7 +97,7 @@ __device__ inline UnitInfo unit_info(const MfmaPrefillArgs& a, int u) {
     seq_geom(a, n, r.q0, r.P, r.L, r.kvo, r.hist);
     const int q_lo = qb * BQ;
     if (q_lo >= r.P) {
-        r.tiles = 0;
+        r.tiles = -1;   // no query rows: no work
         return r;
     }
     int kend = a.causal ? r.hist + min(q_lo + BQ, r.P) : r.L;
@@ -105,68 +106,132 @@ __device__ inline UnitInfo unit_info(const MfmaPrefillArgs& a, int u) {
     return r;
 }
 
-// Units ranked by key tiles (descending, ties by index) for up to kRankUnits
-// units; larger batches keep index order.  Every thread of the work-group
-// calls rank_units (it contains barriers); it leaves in LDS each unit's tiles
-// and lengths (so the chosen unit costs no second global round trip) and the
-// unit at each rank, and returns the split decision: true when the host's key
-// split is dropped because no unit has more key tiles than a compute unit's
-// share of the whole launch (sum of tiles x Hq / CUs).  Such even loads run
-// best unsplit (one work-group per unit, no partials or merge); uneven ones,
-// where the longest unit would set the time, keep the split.
+// The launch's items, from the actual lengths (up to kRankUnits units): the
+// units that have query rows, where the launch has room for partials cut into
+// equal chunks of at most `limit` tiles, and ranked by tiles per chunk
+// (descending, ties by index).  Every work-group derives the same items from the
+// same lengths; item y is the y-th chunk in that order.
+//
+// limit: no unit is cut when the longest has at most a compute unit's share of
+// the launch (sum of tiles x Hq / CUs): such loads run best unsplit (no
+// partials, no merge).  Otherwise the longest is cut into the fewest
+// equal chunks of at most kShare / 8 of a resident slot's share (at least
+// kMinChunkTiles), and the others to the same size.  The launched items and the
+// partial slots bound it too: a cut unit of t tiles has
+// ceil(t / limit) <= t / limit + 1 chunks, at most 2 t / limit, so
+// sum / limit <= extra items and 2 sum / limit <= slots suffice.
+//
+// pick_item leaves in LDS each unit's lengths, so that the chosen unit costs no
+// second global round trip; every thread of the work-group calls it (it contains
+// barriers).
 constexpr int kRankUnits = 1024;
+constexpr int kMinChunkTiles = 8;
+// 14/2/64 eight 512-row fp16 chunks on prefixes up to 4096: 62.6 us at 10 / 8,
+// 62.3 at 12, 58.6 at 14 and 16; the fp32 form 159 .. 160 at all four.
+constexpr int kShare = 14;
 
-__device__ inline bool rank_units(const MfmaPrefillArgs& a, int* order) {
-    __shared__ int s_plan[2];   // sum of the units' tiles, longest unit's tiles
-    const int U = a.N * a.qblocks;
-    if (U > kRankUnits) return false;
-    int* tiles = order;
-    int* at = order + kRankUnits;
-    int* q0s = order + 2 * kRankUnits;
-    int* ps = order + 3 * kRankUnits;
-    int* ls = order + 4 * kRankUnits;
-    int* kvos = order + 5 * kRankUnits;
-    for (int u = threadIdx.x; u < U; u += blockDim.x) {
-        const UnitInfo r = unit_info(a, u);
-        tiles[u] = r.tiles;
-        q0s[u] = r.q0;
-        ps[u] = r.P;
-        ls[u] = r.L;
-        kvos[u] = r.kvo;
-    }
-    __syncthreads();
-    // The rank pass reads every unit's tiles: unit 0's thread also sums them, and
-    // the thread of rank 0 holds the longest.
-    for (int u = threadIdx.x; u < U; u += blockDim.x) {
-        const int tu = tiles[u];
-        int r = 0, sum = 0;
-        for (int v = 0; v < U; ++v) {
-            const int tv = tiles[v];
-            r += (tv > tu) | ((tv == tu) & (v < u));
-            sum += tv;
-        }
-        at[r] = u;
-        if (u == 0) s_plan[0] = sum;
-        if (r == 0) s_plan[1] = tu;
-    }
-    __syncthreads();
-    return a.max_chunks > 1 && (int64_t)s_plan[1] * a.n_cus <= (int64_t)s_plan[0] * a.Hq;
+struct Item {
+    int unit, ci, chunks, part;   // part: partial slot of chunk 0 (chunks > 1)
+};
+
+// Sum over aligned groups of 8 lanes.
+__device__ inline int group8_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, kDppQuadXor1, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppQuadXor2, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowHalfMirror, 0xF, 0xF, false);
+    return v;
 }
 
-// The unit at `rank` (after rank_units) and its UnitInfo.
-__device__ inline int ranked_unit(const MfmaPrefillArgs& a, int rank, const int* order,
-                                  UnitInfo& info) {
-    if (a.N * a.qblocks > kRankUnits) {
-        info = unit_info(a, rank);
-        return rank;
+__device__ inline bool pick_item(const MfmaPrefillArgs& a, int y, int* lds, Item& it, UnitInfo& info) {
+    __shared__ Item s_item;
+    const int U = a.N * a.qblocks;
+    if (U > kRankUnits) {   // index order, nothing cut
+        if (y >= U) return false;
+        it = Item{y, 0, 1, 0};
+        info = unit_info(a, y);
+        return info.tiles >= 0;
     }
-    const int u = order[kRankUnits + rank];
-    info.q0 = order[2 * kRankUnits + u];
-    info.P = order[3 * kRankUnits + u];
-    info.L = order[4 * kRankUnits + u];
-    info.kvo = order[5 * kRankUnits + u];
-    info.tiles = order[u];
-    return u;
+    int* tiles = lds;
+    int* key = lds + kRankUnits;   // tiles per chunk << 12 | chunks; -1: no rows
+    int* q0s = lds + 2 * kRankUnits;
+    int* ps = lds + 3 * kRankUnits;
+    int* ls = lds + 4 * kRankUnits;
+    int* kvos = lds + 5 * kRankUnits;
+    const bool cut = a.max_parts > 0;   // uniform
+    const int U4 = (U + 3) & ~3;
+    for (int u = threadIdx.x; u < U4; u += blockDim.x) {
+        UnitInfo r;
+        r.tiles = -1;
+        if (u < U) {
+            r = unit_info(a, u);
+            q0s[u] = r.q0;
+            ps[u] = r.P;
+            ls[u] = r.L;
+            kvos[u] = r.kvo;
+        }
+        tiles[u] = r.tiles;
+        key[u] = r.tiles < 0 ? -1 : (r.tiles << 12) | 1;
+    }
+    if (threadIdx.x == 0) s_item.unit = -1;
+    __syncthreads();
+    if (cut) {
+        int sum = 0, longest = 0;
+        for (int v = threadIdx.x & 63; v < U; v += 64) {   // every wave for itself
+            const int t = max(tiles[v], 0);
+            sum += t;
+            longest = max(longest, t);
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            sum += __shfl_xor(sum, off, 64);
+            longest = max(longest, __shfl_xor(longest, off, 64));
+        }
+        if ((int64_t)longest * a.n_cus > (int64_t)sum * a.Hq) {   // uniform
+            const int most = max(kMinChunkTiles, (int)ceilf((float)sum * a.chunk_share));
+            const int k = (longest + most - 1) / most;
+            const int limit = max((longest + k - 1) / k, max((2 * sum + a.max_parts - 1) / a.max_parts,
+                                                             (sum + a.extra_items - 1) / a.extra_items));
+            for (int u = threadIdx.x; u < U; u += blockDim.x) {
+                const int t = tiles[u];
+                if (t > limit) {
+                    const int n = (t + limit - 1) / limit;
+                    key[u] = ((t + n - 1) / n) << 12 | n;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    // Eight lanes per unit, each over an eighth of the others.
+    for (int u0 = 0; u0 < U; u0 += blockDim.x / 8) {
+        const int u = u0 + threadIdx.x / 8;
+        const int ku = u < U ? key[u] : -1;
+        int before = 0, parts = 0;   // chunks of the units ranked before u; those of cut units
+        for (int v = 4 * (threadIdx.x & 7); v < U4; v += 32) {
+            const int4 kv = *reinterpret_cast<const int4*>(key + v);
+            const int k4[4] = {kv.x, kv.y, kv.z, kv.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int n = (k4[e] > ku) | ((k4[e] == ku) & (v + e < u)) ? k4[e] & 4095 : 0;
+                before += n;
+                parts += n > 1 ? n : 0;
+            }
+        }
+        before = group8_sum(before);
+        parts = group8_sum(parts);
+        if (u >= U || (threadIdx.x & 7) != 0) continue;
+        const int n = ku < 0 ? 0 : ku & 4095;
+        if (y >= before && y < before + n) s_item = Item{u, y - before, n, parts};
+        if (cut && blockIdx.x == 0) a.table[u] = make_int2(parts, n);   // for the merge kernel
+    }
+    __syncthreads();
+    it = s_item;
+    if (it.unit < 0) return false;
+    info.q0 = q0s[it.unit];
+    info.P = ps[it.unit];
+    info.L = ls[it.unit];
+    info.kvo = kvos[it.unit];
+    info.tiles = tiles[it.unit];
+    return true;
 }
 
 // Wave priority around the S = K Q^T cluster (s_setprio: issue arbitration
@@ -190,21 +255,19 @@ constexpr int kXcds = 8;   // XCDs of an MI355X; work-groups go to them round-ro
 
 // One work-group's work item, from its blockIdx.
 //
-// Work: Y = N x qblocks x max_chunks ranked chunk slots (blockIdx-independent
-// order: slot / max_chunks is a rank in the descending order of the units'
-// key tiles, longest-processing-time first) times Hkv kv-head groups of G
-// q heads, which read the same K/V tiles.  The dispatcher hands consecutive
+// Items (pick_item's order: longest first) times Hkv kv-head groups of G q
+// heads, which read the same K/V tiles.  The dispatcher hands consecutive
 // work-groups to the 8 XCDs in turn, and each XCD has its own L2, so group
-// j (slot-major) goes to XCD j % 8 with its G heads as that XCD's next G
+// j (item-major) goes to XCD j % 8 with its G heads as that XCD's next G
 // work-groups: they run together and share their K/V reads in one L2.
 struct Work {
-    int hq, kvh, unit, n, ci, q0, P, q_lo, L, kvo, hist, kend, t_begin, t_end;
+    int hq, kvh, n, ci, part, q0, P, q_lo, L, kvo, hist, kend, t_begin, t_end;
     bool direct;   // one chunk: write the output row itself
 };
 
 // False when the work-group has nothing to do (uniform over the work-group;
 // it may return before or after the ranking barriers, never between).
-__device__ inline bool take_work(const MfmaPrefillArgs& a, int* order, Work& wk) {
+__device__ inline bool take_work(const MfmaPrefillArgs& a, int* lds, Work& wk) {
     const int G = a.Hq / a.Hkv;
     // Work-groups b, b + CUs, b + 2 CUs of the first resident set share a CU.
     // When a CU holds two or more, the second set takes its items in reverse,
@@ -217,45 +280,28 @@ __device__ inline bool take_work(const MfmaPrefillArgs& a, int* order, Work& wk)
     }
     const int xcd = bid % kXcds, r = bid / kXcds;
     const int j = (r / G) * kXcds + xcd;
-    if (j >= a.groups) return false;
     wk.kvh = j % a.Hkv;
     wk.hq = wk.kvh * G + r % G;
-    const int y = j / a.Hkv;
-    // Every work-group takes the same decision from the same lengths.  Unsplit,
-    // the first N x qblocks chunk slots are the units themselves (chunk 0) and
-    // the other work-groups have nothing to do.
-    const bool unsplit = rank_units(a, order);
-    if (blockIdx.x == 0 && threadIdx.x == 0 && a.plan_flag != nullptr) *a.plan_flag = unsplit ? 1 : 0;
-    int slot;
-    if (unsplit) {
-        if (y >= a.N * a.qblocks) return false;
-        slot = y;
-        wk.ci = 0;
-    } else {
-        slot = y / a.max_chunks;
-        wk.ci = y - slot * a.max_chunks;   // key chunk of the unit
-    }
+    Item it;
     UnitInfo ui;
-    wk.unit = ranked_unit(a, slot, order, ui);  // (sequence, query block)
-    wk.n = wk.unit / a.qblocks;
-    const int qb = a.qblocks - 1 - (wk.unit % a.qblocks);
+    if (!pick_item(a, j / a.Hkv, lds, it, ui)) return false;
+    wk.n = it.unit / a.qblocks;
+    const int qb = a.qblocks - 1 - (it.unit % a.qblocks);
     wk.q0 = ui.q0;
     wk.P = ui.P;
     wk.q_lo = qb * BQ;
-    if (wk.q_lo >= wk.P) return false;
     wk.L = ui.L;
     wk.kvo = ui.kvo;
     wk.hist = a.contig ? 0 : ui.L - ui.P;   // as seq_geom (not kept with the ranked units)
     int kend = a.causal ? wk.hist + min(wk.q_lo + BQ, wk.P) : wk.L;
     wk.kend = kend < 0 ? 0 : (kend > wk.L ? wk.L : kend);
-    const int ntiles = (wk.kend + BN - 1) / BN;
-    // at most max_chunks chunks (a max_seq_len bound below a length): the last
-    // one takes the remaining tiles
-    const int nchunks = unsplit ? 1 : min((ntiles + a.chunk_tiles - 1) / a.chunk_tiles, a.max_chunks);
-    if (wk.ci > 0 && wk.ci >= nchunks) return false;   // chunk 0 also covers an empty key range (zeros)
-    wk.t_begin = wk.ci * a.chunk_tiles;
-    wk.t_end = wk.ci == nchunks - 1 ? ntiles : min(wk.t_begin + a.chunk_tiles, ntiles);
-    wk.direct = nchunks <= 1;
+    // equal chunks; a unit of no tiles has one, which writes zeros
+    const int per = (ui.tiles + it.chunks - 1) / it.chunks;
+    wk.ci = it.ci;
+    wk.part = it.part + it.ci;
+    wk.t_begin = min(it.ci * per, ui.tiles);
+    wk.t_end = min(wk.t_begin + per, ui.tiles);
+    wk.direct = it.chunks == 1;
     return true;
 }
 
@@ -374,7 +420,7 @@ void prefill_mfma_kernel(MfmaPrefillArgs a) {
     // ranking must complete here before any wave writes the first tile.
     if constexpr (CG) lds_barrier();
     poison_uncovered_rows<T, D>(a, wk);
-    const int hq = wk.hq, kvh = wk.kvh, unit = wk.unit, n = wk.n, ci = wk.ci;
+    const int hq = wk.hq, kvh = wk.kvh, n = wk.n;
     const int q0 = wk.q0, P = wk.P, q_lo = wk.q_lo, L = wk.L, kend = wk.kend;
     const int t_begin = wk.t_begin, t_end = wk.t_end;
     const bool direct = wk.direct;
@@ -742,7 +788,7 @@ void prefill_mfma_kernel(MfmaPrefillArgs a) {
     // (one chunk: the output row; several: an fp32 partial row + log2-sum-exp2,
     // -inf for a row that saw no key of this chunk)
     T* og = reinterpret_cast<T*>(a.out);
-    const int64_t pidx = ((int64_t)unit * a.max_chunks + ci) * a.Hq + hq;
+    const int64_t pidx = (int64_t)wk.part * a.Hq + hq;
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
         const float lt = osum[nt][0];
@@ -827,7 +873,7 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
     // ranking must complete here before any wave writes the first tile.
     if constexpr (CG) lds_barrier();
     poison_uncovered_rows<float, D>(a, wk);
-    const int hq = wk.hq, kvh = wk.kvh, unit = wk.unit, n = wk.n, ci = wk.ci;
+    const int hq = wk.hq, kvh = wk.kvh, n = wk.n;
     const int q0 = wk.q0, P = wk.P, q_lo = wk.q_lo, L = wk.L, kend = wk.kend;
     const int t_begin = wk.t_begin, t_end = wk.t_end;
     const int last_page = L > 0 ? (L - 1) / kPage : 0;
@@ -1080,7 +1126,7 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
     }
 
     float* og = reinterpret_cast<float*>(a.out);
-    const int64_t pidx = ((int64_t)unit * a.max_chunks + ci) * a.Hq + hq;
+    const int64_t pidx = (int64_t)wk.part * a.Hq + hq;
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
         float lt = lsum[nt];
@@ -1262,7 +1308,7 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
     // its own barrier).
     if constexpr (CG) lds_barrier();
     poison_uncovered_rows<float, D>(a, wk);
-    const int hq = wk.hq, kvh = wk.kvh, unit = wk.unit, n = wk.n, ci = wk.ci;
+    const int hq = wk.hq, kvh = wk.kvh, n = wk.n;
     const int q0 = wk.q0, P = wk.P, q_lo = wk.q_lo, L = wk.L, kend = wk.kend;
     const int t_begin = wk.t_begin, t_end = wk.t_end;
     const int last_page = L > 0 ? (L - 1) / kPage : 0;
@@ -1625,7 +1671,7 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
     lsum += __shfl_xor(lsum, 32, 64);
     if (ql >= P) return;
     const float inv = lsum > 0.f ? 1.0f / (kScaleV * lsum) : 0.f;
-    const int64_t prow = (((int64_t)unit * a.max_chunks + ci) * a.Hq + hq) * BQ + w * WQ + c32;
+    const int64_t prow = ((int64_t)wk.part * a.Hq + hq) * BQ + w * WQ + c32;
     float* drow = wk.direct ? reinterpret_cast<float*>(a.out) + ((int64_t)(q0 + ql) * a.Hq + hq) * D
                             : a.part_o + prow * D;
 #pragma unroll
@@ -1656,26 +1702,22 @@ __device__ inline void store4<float>(float* p, float x, float y, float z, float 
 // log-sum-exp (each chunk's lse and row slice are loaded together).
 template <typename T, int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(MfmaPrefillArgs a) {
-    // The main kernel's split decision; loaded together with the lengths below
-    // and checked before anything is read or written.
-    const int unsplit = *a.plan_flag;
     constexpr int TPR = 256 / BQ;     // threads per row
     constexpr int V4 = D / TPR / 4;   // float4 per thread
     const int hq = blockIdx.x, unit = blockIdx.y;
+    // The unit's first partial slot and chunks, from the main kernel; loaded
+    // together with the lengths below and checked before anything is written.
+    const int2 cut = a.table[unit];
     const int n = unit / a.qblocks;
     const int qb = a.qblocks - 1 - (unit % a.qblocks);
     int q0, P, L, kvo, hist;
     seq_geom(a, n, q0, P, L, kvo, hist);
-    if (unsplit != 0) return;   // every row was written by the main kernel
+    const int nchunks = cut.y;
+    if (nchunks <= 1) return;   // written directly (or no rows)
     const int q_lo = qb * BQ;
     const int row = threadIdx.x / TPR, part = threadIdx.x % TPR;
     if (q_lo + row >= P) return;
-    int kend = a.causal ? hist + min(q_lo + BQ, P) : L;
-    kend = kend < 0 ? 0 : (kend > L ? L : kend);
-    const int ntiles = (kend + BN - 1) / BN;
-    const int nchunks = min((ntiles + a.chunk_tiles - 1) / a.chunk_tiles, a.max_chunks);   // as take_work
-    if (nchunks <= 1) return;   // written directly
-    const int64_t p0 = ((int64_t)unit * a.max_chunks) * a.Hq + hq;   // chunk c at p0 + c * Hq
+    const int64_t p0 = (int64_t)cut.x * a.Hq + hq;   // chunk c at p0 + c * Hq
     float M = -INFINITY, W = 0.0f;
     float4 acc[V4];
 #pragma unroll
@@ -1731,20 +1773,20 @@ bool prefill_mfma_handles(int head_dim, int block_size, int dtype) {
     return block_size == kPage && (head_dim == 64 || head_dim == 96 || head_dim == 128 || head_dim == 256);
 }
 
-// Key-range split.  When the (sequence, query block, q head) units alone
-// would leave the GPU idle, a unit's key tiles are cut into chunks of
-// ceil(max_tiles / k) tiles, k chosen so that the launch offers about kFill
-// work-groups per resident slot (counted as if every unit had the longest key
-// range), with chunks of at least kMinChunkTiles tiles.  With enough units
-// (k = 1) nothing is split: no partials and no merge.  The workspace is sized
-// from the shape alone, for kSizingSlots resident slots (256 CUs x 4
-// work-groups, above what this kernel reaches); a launch takes the smaller of
-// that k and the one of its device's actual resident count.  About one
-// work-group per slot: with fp32 partials, configuration 4 runs two chunks
-// per long unit at 58.1 us against 59.8 us for three (1.5 per slot) and
-// 80 us for two per slot; the fewer chunks, the less partial traffic.
-constexpr double kFill = 1.0;
-constexpr int kMinChunkTiles = 8;
+// Key-range split (pick_item).  The host lets a launch cut units, which costs a
+// merge kernel and the partials' traffic, when the units' heads alone would not
+// fill the resident slots.  With more, cutting measured slower even where one
+// unit is far longer than the others (32/8/128 bf16 chunks of 1 .. 1101 rows on
+// prefixes up to 3000: 81 us, cut 86 .. 97).  Units are counted from the rows
+// (at most total_q / BQ + N hold any), not as N x the longest sequence's blocks:
+// 28/4/128 bf16 chunks of 64, 31, 700 and 5 rows 89 -> 38 us by that count.
+// Kernels of one work-group per CU (fp32 at head_dim 96 / 128, head_dim 256) cut
+// up to twice their slots: no second work-group runs beside a long one there
+// (32/8/128 fp32 chunks of 512, 300, 77 on 1000, 0, 2000: 288 heads' units, 169 ->
+// 120 us).
+// The workspace is sized for kSizingSlots resident slots (256 CUs x 4
+// work-groups, above what these kernels reach), so that it does not depend on
+// the device.
 constexpr int kSizingSlots = 1024;
 
 typedef void (*PrefillFn)(MfmaPrefillArgs);
@@ -1796,43 +1838,42 @@ PrefillFn merge_kernel(int dtype, int head_dim) {
     return merge_for<bf16_t>(head_dim);
 }
 
-// Workspace header: the main kernel's split decision (one int), read by the
-// merge kernel.
+// Workspace: a header, then max_parts partial slots (Hq x BQ rows each), then one
+// slot for the merge kernel's table.
 constexpr size_t kPlanHeaderBytes = 256;
 
 struct ChunkPlan {
-    int qblocks, max_chunks, chunk_tiles;
+    int qblocks, units;   // query blocks per sequence; bound of the units with rows
+    int extra, parts;     // items beyond `units`; partial slots (0: nothing is cut)
 };
 
-// slots <= 0: size for kSizingSlots; otherwise the launch plan for that many
-// resident slots (never more chunks than the sizing plan).
-ChunkPlan chunk_plan(int N, int Hq, int total_q, int max_q_len, int max_seq_len, int slots) {
+ChunkPlan chunk_plan(int N, int Hq, int total_q, int max_q_len, int max_seq_len) {
     ChunkPlan c;
     const int qmax = (max_q_len > 0 && max_q_len < total_q) ? max_q_len : total_q;
     c.qblocks = (qmax + BQ - 1) / BQ;
+    const int64_t all = (int64_t)N * c.qblocks;
+    c.units = (int)std::min<int64_t>(all, (int64_t)total_q / BQ + N);   // sum of ceil(rows / BQ)
     const int max_tiles = (std::max(max_seq_len, 1) + BN - 1) / BN;
-    const double unit_heads = (double)N * c.qblocks * Hq;
-    auto splits = [&](int s) {
-        int k = (int)std::ceil(kFill * s / unit_heads);
-        k = std::min(k, std::max(1, max_tiles / kMinChunkTiles));
-        return std::max(k, 1);
-    };
-    int k = splits(kSizingSlots);
-    if (slots > 0) k = std::min(k, splits(slots));
-    c.chunk_tiles = (max_tiles + k - 1) / k;
-    c.max_chunks = (max_tiles + c.chunk_tiles - 1) / c.chunk_tiles;
+    c.extra = c.parts = 0;
+    if (all <= kRankUnits && max_tiles >= 2 * kMinChunkTiles &&
+        (int64_t)c.units * Hq < kSizingSlots) {
+        // sum / limit at the share, and a quarter more for the equal chunks
+        const int64_t share = (kSizingSlots * 10 + Hq * kShare - 1) / (Hq * kShare);
+        c.extra = (int)std::max<int64_t>(1, share);
+        c.parts = (int)std::max<int64_t>(2, std::min<int64_t>(2 * share, (int64_t)c.units * (max_tiles / kMinChunkTiles + 1)));
+    }
     return c;
 }
+
+size_t part_bytes(int Hq, int head_dim) { return (size_t)Hq * BQ * (1 + head_dim) * sizeof(float); }
 
 }  // namespace
 
 size_t prefill_mfma_workspace(int N, int Hq, int head_dim, int block_size, int dtype, int total_q,
                               int max_q_len, int max_seq_len) {
     if (!prefill_mfma_handles(head_dim, block_size, dtype) || N <= 0 || total_q <= 0) return 0;
-    const ChunkPlan c = chunk_plan(N, Hq, total_q, max_q_len, max_seq_len, 0);
-    if (c.max_chunks <= 1) return 0;
-    const size_t parts = (size_t)N * c.qblocks * c.max_chunks * Hq;
-    return kPlanHeaderBytes + parts * BQ * sizeof(float) + parts * BQ * head_dim * sizeof(float);
+    const ChunkPlan c = chunk_plan(N, Hq, total_q, max_q_len, max_seq_len);
+    return c.parts > 0 ? kPlanHeaderBytes + (size_t)(c.parts + 1) * part_bytes(Hq, head_dim) : 0;
 }
 
 int launch_prefill_mfma(MfmaPrefillArgs a, int head_dim, int block_size, int dtype,
@@ -1841,36 +1882,37 @@ int launch_prefill_mfma(MfmaPrefillArgs a, int head_dim, int block_size, int dty
     if (!prefill_mfma_handles(head_dim, block_size, dtype)) return -1;
     if (((uintptr_t)a.q | (uintptr_t)a.out | (uintptr_t)a.k | (uintptr_t)a.v) & 15) return -1;
     const int slots = resident_workgroups(reinterpret_cast<const void*>(prefill_kernel(dtype, head_dim, false)), 256);
-    const ChunkPlan c = chunk_plan(a.N, a.Hq, total_q, max_q_len, max_seq_len, slots);
-    a.qblocks = c.qblocks;
-    const size_t need = prefill_mfma_workspace(a.N, a.Hq, head_dim, block_size, dtype, total_q,
-                                               max_q_len, max_seq_len);
-    if (c.max_chunks > 1 && workspace != nullptr && workspace_bytes >= need) {
-        // partials laid out for the sizing plan's chunk count (>= this plan's)
-        const ChunkPlan z = chunk_plan(a.N, a.Hq, total_q, max_q_len, max_seq_len, 0);
-        const size_t parts = (size_t)a.N * z.qblocks * z.max_chunks * a.Hq;
-        a.max_chunks = c.max_chunks;
-        a.chunk_tiles = c.chunk_tiles;
-        char* base = reinterpret_cast<char*>(workspace);
-        a.plan_flag = reinterpret_cast<int*>(base);
-        a.part_lse = reinterpret_cast<float*>(base + kPlanHeaderBytes);
-        a.part_o = reinterpret_cast<float*>(base + kPlanHeaderBytes + parts * BQ * sizeof(float));
-    } else {   // no split, or no (or too small a) workspace: one chunk per unit
-        a.max_chunks = 1;
-        a.chunk_tiles = 1 << 30;
-        a.part_lse = nullptr;
-        a.part_o = nullptr;
-        a.plan_flag = nullptr;
-    }
     a.n_cus = device_cus();
     a.resident = a.contig ? resident_workgroups(reinterpret_cast<const void*>(prefill_kernel(dtype, head_dim, true)), 256)
                           : slots;
-    a.groups = a.N * a.qblocks * a.max_chunks * a.Hkv;
+    const ChunkPlan c = chunk_plan(a.N, a.Hq, total_q, max_q_len, max_seq_len);
+    a.qblocks = c.qblocks;
+    const size_t need = prefill_mfma_workspace(a.N, a.Hq, head_dim, block_size, dtype, total_q,
+                                               max_q_len, max_seq_len);
+    a.max_parts = 0;
+    a.extra_items = 0;
+    a.table = nullptr;
+    a.part_lse = a.part_o = nullptr;
+    const int cut_below = a.resident < 2 * a.n_cus ? 2 * a.resident : a.resident;
+    if (need > 0 && (int64_t)c.units * a.Hq < cut_below && workspace != nullptr &&
+        workspace_bytes >= need) {
+        a.max_parts = c.parts;
+        a.extra_items = c.extra;
+        a.chunk_share = (float)kShare / 8.0f * a.Hq / std::min(a.resident, kSizingSlots);
+        char* base = reinterpret_cast<char*>(workspace) + kPlanHeaderBytes;
+        const size_t rows = (size_t)c.parts * a.Hq * BQ;
+        a.part_lse = reinterpret_cast<float*>(base);
+        a.part_o = a.part_lse + rows;
+        a.table = reinterpret_cast<int2*>(base + (size_t)c.parts * part_bytes(a.Hq, head_dim));
+    }
+    // every unit's own item (index order above kRankUnits units), and the cuts
+    const int64_t all = (int64_t)a.N * a.qblocks;
+    const int64_t groups = (all > kRankUnits ? all : c.units + a.extra_items) * a.Hkv;
     const int G = a.Hq / a.Hkv;
-    dim3 grid((unsigned)(((a.groups + kXcds - 1) / kXcds) * kXcds * G));
-    dim3 mgrid(a.Hq, a.N * a.qblocks);
+    dim3 grid((unsigned)(((groups + kXcds - 1) / kXcds) * kXcds * G));
     prefill_kernel(dtype, head_dim, a.contig != 0)<<<grid, 256, 0, st>>>(a);
-    if (a.max_chunks > 1) merge_kernel(dtype, head_dim)<<<mgrid, 256, 0, st>>>(a);
+    if (a.max_parts > 0)
+        merge_kernel(dtype, head_dim)<<<dim3(a.Hq, a.N * a.qblocks), 256, 0, st>>>(a);
     return check_launch(a.contig ? "llkv_first_prefill_batched" : "llkv_paged_prefill");
 }
 

@@ -114,3 +114,55 @@ def test_prefill_f32_split_terms(case, d):
         assert torch.equal(out[~fine], ref[~fine]), (case, name)
         err = (out - ref)[fine].abs()
         assert torch.all(err <= 1e-6 * unit + 1e-5 * ref[fine].abs()), (case, name, float(err.max()))
+
+
+# Work items of a prefill launch: (prefixes, chunks) with cut key ranges (one long sequence: many
+# chunks; several of uneven length; the merge's rows past a chunk's query rows), more units than
+# the ranking's 32 per pass, more than it ranks at all, and sequences without rows or keys.
+def _items(name):
+    g = torch.Generator().manual_seed(11)
+    if name == "one_long":
+        return 4, 2, [40000], [5]
+    if name == "uneven":
+        return 4, 2, [6000, 0, 1500, 16], [3, 140, 129, 1]
+    if name == "units_300":
+        return 2, 1, torch.randint(0, 900, (300,), generator=g).tolist(), torch.randint(0, 3, (300,), generator=g).tolist()
+    if name == "units_1100":
+        return 2, 1, torch.randint(0, 90, (1100,), generator=g).tolist(), torch.randint(0, 3, (1100,), generator=g).tolist()
+    return 4, 2, [0, -7, 2000, 0, -64], [0, 7, 130, 40, 64]   # "no_keys": keys = prefix + chunk = 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("name", ["one_long", "uneven", "units_300", "units_1100", "no_keys"])
+def test_prefill_work_items(name, dtype):
+    g = torch.Generator().manual_seed(12)
+    d = 64
+    hq, hkv, prefixes, chunks = _items(name)
+    totals = [p + c for p, c in zip(prefixes, chunks)]
+    need = [(n + 15) // 16 for n in totals]
+    nb = sum(need) + 1
+    kp = torch.randn(nb, 16, hkv, d, generator=g).to(dtype)
+    vp = torch.randn(nb, 16, hkv, d, generator=g).to(dtype)
+    q = torch.randn(sum(chunks), hq, d, generator=g).to(dtype)
+    perm = torch.randperm(nb, generator=g).to(torch.int32)
+    table = torch.full((len(chunks), max(need)), -1, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = perm[at:at + n]
+        at += n
+    cu = torch.tensor([0] + torch.tensor(chunks).cumsum(0).tolist(), dtype=torch.int32)
+    out = kc.paged_prefill(q.to(DEV), kp.to(DEV), vp.to(DEV), table.to(DEV), cu.to(DEV),
+                           torch.tensor(totals, dtype=torch.int32, device=DEV), max(chunks), max(totals)).cpu().double()
+    for i, (n, c) in enumerate(zip(totals, chunks)):
+        if c == 0:
+            continue
+        got = out[cu[i]:cu[i + 1]]
+        if n == 0:
+            assert torch.all(got == 0), i
+            continue
+        rows = table[i, :need[i]].long()
+        k, v = (p[rows].reshape(-1, hkv, d)[:n] for p in (kp, vp))
+        ref = _attend64(q[cu[i]:cu[i + 1]], k, v, n - c)
+        bar = 2e-3 * (ref.abs() + ref.square().mean(-1, keepdim=True).sqrt()) if dtype == torch.float16 else \
+            1e-6 + 1e-5 * ref.abs()
+        assert torch.all((got - ref).abs() <= bar), (i, float(((got - ref).abs() / bar).max()))
