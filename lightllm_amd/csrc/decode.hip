@@ -139,12 +139,15 @@ __global__ __launch_bounds__(64) void decode_generic_kernel(DecodeArgs a) {
 // pl[j * pl_step]; live(j) false skips an entry.  One wave; lane owns dims
 // lane + 64 i; entries are fetched kMergeBatch at a time with a running
 // maximum, so a merge costs ceil(count / kMergeBatch) memory round trips.
+// kMergeBatch: 16 for fixed splits (up to 16 partials in one trip), 4 for the
+// balanced schedule, whose units are mostly cut in two or three (16 issues up to
+// 64 masked loads a lane for them): 61 x 100 .. 2100 tokens of 16/8/256 bf16 120
+// -> 106 us a call, 256 lognormal contexts of 32/8/128 fp16 388 -> 385; 2 and 8
+// measured the same as 4.
 // The reference's paged_attention_reduce_kernel
 // (src/kv_cache/paged_attention.cu:477-532) computes the same sum in
 // unnormalised form: out = sum_j 2^(lse_j - M) o_j / sum_j 2^(lse_j - M).
-constexpr int kMergeBatch = 16;
-
-template <typename T, int MD, class Live>
+template <typename T, int MD, int kMergeBatch, class Live>
 __device__ inline void merge_partials(const float* po, int64_t po_step, const float* pl,
                                       int64_t pl_step, int count, int D, Live live, T* out) {
     const int lane = threadIdx.x & 63;
@@ -197,7 +200,7 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(DecodeArgs a) {
     const SplitGeo geo = split_geo(a, b);
     if (geo.nsplit <= 1) return;   // written directly by the split kernel
     const int64_t bh = (int64_t)b * a.Hq + hq;
-    merge_partials<T, MD>(a.part_o + bh * a.S_max * a.D, a.D, a.part_lse + bh * a.S_max, 1,
+    merge_partials<T, MD, 16>(a.part_o + bh * a.S_max * a.D, a.D, a.part_lse + bh * a.S_max, 1,
                           geo.nsplit, a.D, AllLive(), reinterpret_cast<T*>(a.out) + bh * a.D);
 }
 
@@ -234,9 +237,9 @@ __global__ __launch_bounds__(1024) void decode_merge_balanced_kernel(DecodeArgs 
     const float* pl = a.part_lse + seg0 * G + h;
     const int cnt = (int)(wl - wf + 1);
     if (T_ >= a.nwg)   // every work-group holds pages: all entries live
-        merge_partials<T, MD>(po, (int64_t)G * D, pl, G, cnt, D, AllLive(), out);
+        merge_partials<T, MD, 4>(po, (int64_t)G * D, pl, G, cnt, D, AllLive(), out);
     else
-        merge_partials<T, MD>(po, (int64_t)G * D, pl, G, cnt, D, LiveWG{wf, T_, a.nwg}, out);
+        merge_partials<T, MD, 4>(po, (int64_t)G * D, pl, G, cnt, D, LiveWG{wf, T_, a.nwg}, out);
 }
 
 // ---------------------------------------------------------------------------

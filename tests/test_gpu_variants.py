@@ -166,3 +166,34 @@ def test_prefill_work_items(name, dtype):
         bar = 2e-3 * (ref.abs() + ref.square().mean(-1, keepdim=True).sqrt()) if dtype == torch.float16 else \
             1e-6 + 1e-5 * ref.abs()
         assert torch.all((got - ref).abs() <= bar), (i, float(((got - ref).abs() / bar).max()))
+
+
+# Balanced decode: a unit cut into exactly the merge's four entries per trip, fewer, more, and many
+# (one sequence of nearly all pages), beside short sequences inside one share.
+@pytest.mark.parametrize("d,hq,hkv", [(64, 14, 2), (128, 32, 8), (256, 16, 8)])
+@pytest.mark.parametrize("long", [2000, 9000, 30000])
+def test_balanced_merge_entries(long, d, hq, hkv):
+    g = torch.Generator().manual_seed(long + d)
+    B = 520 // hkv
+    lens = torch.randint(1, 200, (B,), generator=g).tolist()
+    lens[B // 2] = long
+    assert kc.decode_schedule(B, hq, hkv, d, long, torch.float16)[0] == "balanced"
+    need = [(n + 15) // 16 for n in lens]
+    nb = sum(need)
+    kp = torch.randn(nb, 16, hkv, d, generator=g).half()
+    vp = torch.randn(nb, 16, hkv, d, generator=g).half()
+    q = torch.randn(B, hq, d, generator=g).half()
+    perm = torch.randperm(nb, generator=g).to(torch.int32)
+    table = torch.full((B, max(need)), -1, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = perm[at:at + n]
+        at += n
+    out = kc.paged_decode(q.to(DEV), kp.to(DEV), vp.to(DEV), table.to(DEV),
+                          torch.tensor(lens, dtype=torch.int32, device=DEV), long).cpu().double()
+    for i in (0, 1, B // 2 - 1, B // 2, B // 2 + 1, B - 1):
+        rows = table[i, :need[i]].long()
+        k, v = (p[rows].reshape(-1, hkv, d)[:lens[i]] for p in (kp, vp))
+        ref = _attend64(q[i:i + 1], k, v, lens[i] - 1)[0]
+        bar = 2e-3 * (ref.abs() + ref.square().mean(-1, keepdim=True).sqrt())
+        assert torch.all((out[i] - ref).abs() <= bar), (i, float(((out[i] - ref).abs() / bar).max()))
