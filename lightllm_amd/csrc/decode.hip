@@ -245,8 +245,22 @@ __global__ __launch_bounds__(1024) void decode_merge_balanced_kernel(DecodeArgs 
 // ---------------------------------------------------------------------------
 // Host dispatch
 // ---------------------------------------------------------------------------
+// K/V bytes (by the shape bounds) from which a batch is read with streaming
+// loads: three quarters of the 256 MB last-level cache.  Such a batch finds
+// nothing of itself there on the next call, and loads that do not allocate run
+// faster (256 lognormal contexts of 32/8/128 fp16 390 -> 365 us, 16 x 32768 of
+// 14/2/64 fp16 56 -> 53, 61 x 100 .. 2100 of 16/8/256 bf16 106 -> 99); smaller
+// batches may stay cached (64 x 129 .. 2049 of 14/2/64 fp32, 134 MB: 23.6 us, by
+// streaming loads 24.6).
+constexpr int64_t kStreamBytes = 192ll << 20;
+
 // The tuned kernels of a pool type, plain or fused-append (decode_tuned_*.hip).
-Kernels pick_tuned(int dtype, int D, int G, bool append) {
+Kernels pick_tuned(int dtype, int D, int G, bool append, bool stream = false) {
+    if (stream) {
+        if (dtype == LLKV_DTYPE_F32) return tuned_kernels_f32_stream(D, G, append);
+        if (dtype == LLKV_DTYPE_F16) return tuned_kernels_f16_stream(D, G, append);
+        if (dtype == LLKV_DTYPE_BF16) return tuned_kernels_bf16_stream(D, G, append);
+    }
     if (dtype == LLKV_DTYPE_F32) return tuned_kernels_f32(D, G, append);
     if (dtype == LLKV_DTYPE_F16) return tuned_kernels_f16(D, G, append);
     if (dtype == LLKV_DTYPE_BF16) return tuned_kernels_bf16(D, G, append);
@@ -529,14 +543,15 @@ int paged_decode_impl(const char* fn, void* out, const void* q, const void* k_ne
                          ((size_t)num_kv_heads * head_dim * es) % 16 == 0;
     Kernels ks;
     if (block_size == kPage && aligned) {
-        ks = pick_tuned(dtype, head_dim, G, k_new != nullptr);
+        const bool stream_kv = (int64_t)num_seqs * max_seq_len * num_kv_heads * head_dim * 2 * (int64_t)es > kStreamBytes;
+        ks = pick_tuned(dtype, head_dim, G, k_new != nullptr, stream_kv);
     }
     const int max_pages_hint = (max_seq_len + block_size - 1) / block_size;
     bool balanced = false, wide = false;
-    // The fused-append call takes the plain call's schedule (from the plain
-    // kernels' resident counts), so that its results equal append + decode
-    // bit for bit.
-    const Kernels sched = (k_new != nullptr && ks.split != nullptr) ? pick_tuned(dtype, head_dim, G, false) : ks;
+    // Every call takes the schedule of the plain kernels (from their resident
+    // counts), so that a fused append's results equal append + decode bit for bit
+    // and the loads' form changes no result.
+    const Kernels sched = ks.split != nullptr ? pick_tuned(dtype, head_dim, G, false) : ks;
     decide_schedule(sched, num_seqs, num_kv_heads, block_size, max_seq_len, num_splits, balanced, wide);
 
     DecodeArgs a;

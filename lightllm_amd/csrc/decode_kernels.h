@@ -26,5 +26,9 @@ struct Kernels {
 Kernels tuned_kernels_f32(int D, int G, bool append);
 Kernels tuned_kernels_f16(int D, int G, bool append);
 Kernels tuned_kernels_bf16(int D, int G, bool append);
+// The same kernels with streaming (nontemporal) loads of K and V.
+Kernels tuned_kernels_f32_stream(int D, int G, bool append);
+Kernels tuned_kernels_f16_stream(int D, int G, bool append);
+Kernels tuned_kernels_bf16_stream(int D, int G, bool append);
 
 }  // namespace llkv

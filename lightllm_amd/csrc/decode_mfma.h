@@ -46,6 +46,13 @@ typedef short ms16x4 __attribute__((ext_vector_type(4)));
 
 typedef __bf16 mbf16x8 __attribute__((ext_vector_type(8)));
 
+// A load of K / V, streaming (nontemporal) or not.
+template <bool NT, typename V>
+__device__ inline V load_vec(const void* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+    else return *reinterpret_cast<const V*>(p);
+}
+
 // Score operands S^T = K Q^T per element type.  load_q fills the Q^T operand
 // of query column c (zero beyond G), load_k the K operand of token row c of a
 // page, scores returns the lane's 4 scores scaled into the exp2 domain.
@@ -68,9 +75,10 @@ template <int D> struct ScoreOps<float, D> {
         }
     }
     // krow: K row of the lane's token, at this kv head's dims
+    template <bool NT>
     __device__ static void load_k(const float* krow, int g, KReg (&k)[NK]) {
 #pragma unroll
-        for (int cc = 0; cc < NK; ++cc) k[cc] = *reinterpret_cast<const float4*>(krow + 16 * cc + 4 * g);
+        for (int cc = 0; cc < NK; ++cc) k[cc] = __builtin_bit_cast(float4, load_vec<NT, mu32x4>(krow + 16 * cc + 4 * g));
     }
     // From head_dim 128 on, the four quarters of the head dims accumulate
     // apart and are added pairwise at the end: a quarter of the rounding steps
@@ -96,7 +104,8 @@ template <int D> struct ScoreOps<float, D> {
         else return (acc[0] + acc[1]) + (acc[2] + acc[3]);
     }
     // V[row][dims 4c .. 4c+3] widened to fp32
-    __device__ static float4 load_v4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+    template <bool NT>
+    __device__ static float4 load_v4(const float* p) { return __builtin_bit_cast(float4, load_vec<NT, mu32x4>(p)); }
 };
 
 template <typename T16, int D> struct ScoreOps16 {
@@ -109,9 +118,10 @@ template <typename T16, int D> struct ScoreOps16 {
         for (int ks = 0; ks < NQ; ++ks)
             q[ks] = valid ? *reinterpret_cast<const mu32x4*>(qrow + 32 * ks + 8 * g) : mu32x4{0u, 0u, 0u, 0u};
     }
+    template <bool NT>
     __device__ static void load_k(const T16* krow, int g, KReg (&k)[NK]) {
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks) k[ks] = *reinterpret_cast<const mu32x4*>(krow + 32 * ks + 8 * g);
+        for (int ks = 0; ks < NK; ++ks) k[ks] = load_vec<NT, mu32x4>(krow + 32 * ks + 8 * g);
     }
     __device__ static mf32x4 mma(const mu32x4& a, const mu32x4& b, mf32x4 c) {
         if constexpr (Elem<T16>::kDtype == LLKV_DTYPE_F16)
@@ -125,8 +135,9 @@ template <typename T16, int D> struct ScoreOps16 {
         for (int ks = 0; ks < NK; ++ks) s = mma(k[ks], q[ks], s);
         return s * scale;
     }
+    template <bool NT>
     __device__ static float4 load_v4(const T16* p) {
-        const mu32x2 w = *reinterpret_cast<const mu32x2*>(p);
+        const mu32x2 w = load_vec<NT, mu32x2>(p);
         float f[4];
         if constexpr (sizeof(T16) == 2 && Elem<T16>::kDtype == LLKV_DTYPE_F16) {
             unpack_h2(w.x, f);
@@ -147,7 +158,9 @@ template <int D> struct ScoreOps<bf16_t, D> : ScoreOps16<bf16_t, D> {};
 // loop has no trace of it.
 // WV: waves per work-group (kDecodeWaves; kUnitWaves for the one-work-group-
 // per-unit schedule of small batches).
-template <typename TT, int D, int G, bool A = false, int WV = kDecodeWaves>
+// NT: K and V by nontemporal loads, for batches beyond the last-level cache
+// (kStreamBytes, decode.hip).
+template <typename TT, int D, int G, bool A = false, int WV = kDecodeWaves, bool NT = false>
 struct MfmaDecode {
     static_assert(G >= 1 && G <= 16, "up to 16 query heads per KV head");
     static_assert(D % 32 == 0, "head_dim multiple of 32");
@@ -293,7 +306,7 @@ struct MfmaDecode {
             const int64_t nrow = ((int64_t)sb * a.Hkv + skvh) * D;   // the new rows' offset
             const T* kp = reinterpret_cast<const T*>(a.k) + (int64_t)skvh * D + (phys * kPage + c) * row_elems;
             if (newpage && c == snew_r) kp = reinterpret_cast<const T*>(a.knew) + nrow;
-            Ops::load_k(kp, g, kr);
+            Ops::template load_k<NT>(kp, g, kr);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const T* vp = reinterpret_cast<const T*>(a.v) + (int64_t)skvh * D +
@@ -305,9 +318,9 @@ struct MfmaDecode {
                         vh[h][i] = mu32x2{0u, 0u};
                         vr[h][i] = make_float4(0.f, 0.f, 0.f, 0.f);
                     } else if constexpr (kHalfPV) {
-                        vh[h][i] = *reinterpret_cast<const mu32x2*>(vp + 64 * h);
+                        vh[h][i] = load_vec<NT, mu32x2>(vp + 64 * h);
                     } else {
-                        vr[h][i] = Ops::load_v4(vp + 64 * h);
+                        vr[h][i] = Ops::template load_v4<NT>(vp + 64 * h);
                     }
                 }
             }

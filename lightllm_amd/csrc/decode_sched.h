@@ -109,50 +109,50 @@ Kernels kernels_of() {
 // head_dim 64 / 128 also get the unit schedule's kUnitWaves-wave kernel,
 // except fp32 at head_dim 128, whose body does not fit the 128 registers of
 // four waves per SIMD (~50 would spill).
-template <typename T, int D, int G, bool A>
+template <typename T, int D, int G, bool A, bool NT>
 Kernels kernels_with_unit() {
-    Kernels k = kernels_of<MfmaDecode<T, D, G, A>>();
+    Kernels k = kernels_of<MfmaDecode<T, D, G, A, kDecodeWaves, NT>>();
     if constexpr (!(Elem<T>::kDtype == LLKV_DTYPE_F32 && D == 128))
-        k.unit = decode_split_kernel<MfmaDecode<T, D, G, A, kUnitWaves>>;
+        k.unit = decode_split_kernel<MfmaDecode<T, D, G, A, kUnitWaves, NT>>;
     return k;
 }
 
-template <typename T, int D, bool A>
+template <typename T, int D, bool A, bool NT>
 Kernels tuned_g(int G) {
     switch (G) {
-        case 1: return kernels_with_unit<T, D, 1, A>();
-        case 2: return kernels_with_unit<T, D, 2, A>();
-        case 3: return kernels_with_unit<T, D, 3, A>();
-        case 4: return kernels_with_unit<T, D, 4, A>();
-        case 5: return kernels_with_unit<T, D, 5, A>();
-        case 6: return kernels_with_unit<T, D, 6, A>();
-        case 7: return kernels_with_unit<T, D, 7, A>();
-        case 8: return kernels_with_unit<T, D, 8, A>();
-        case 12: return kernels_with_unit<T, D, 12, A>();
-        case 16: return kernels_with_unit<T, D, 16, A>();
+        case 1: return kernels_with_unit<T, D, 1, A, NT>();
+        case 2: return kernels_with_unit<T, D, 2, A, NT>();
+        case 3: return kernels_with_unit<T, D, 3, A, NT>();
+        case 4: return kernels_with_unit<T, D, 4, A, NT>();
+        case 5: return kernels_with_unit<T, D, 5, A, NT>();
+        case 6: return kernels_with_unit<T, D, 6, A, NT>();
+        case 7: return kernels_with_unit<T, D, 7, A, NT>();
+        case 8: return kernels_with_unit<T, D, 8, A, NT>();
+        case 12: return kernels_with_unit<T, D, 12, A, NT>();
+        case 16: return kernels_with_unit<T, D, 16, A, NT>();
     }
     return Kernels();
 }
 
 // head_dim 96 (Phi-3 layouts) and 256 (Gemma-2 / Gemma-3 layouts): group
 // sizes 1, 2, 4, 8.
-template <typename T, int D, bool A>
+template <typename T, int D, bool A, bool NT>
 Kernels tuned_g_few(int G) {
     switch (G) {
-        case 1: return kernels_of<MfmaDecode<T, D, 1, A>>();
-        case 2: return kernels_of<MfmaDecode<T, D, 2, A>>();
-        case 4: return kernels_of<MfmaDecode<T, D, 4, A>>();
-        case 8: return kernels_of<MfmaDecode<T, D, 8, A>>();
+        case 1: return kernels_of<MfmaDecode<T, D, 1, A, kDecodeWaves, NT>>();
+        case 2: return kernels_of<MfmaDecode<T, D, 2, A, kDecodeWaves, NT>>();
+        case 4: return kernels_of<MfmaDecode<T, D, 4, A, kDecodeWaves, NT>>();
+        case 8: return kernels_of<MfmaDecode<T, D, 8, A, kDecodeWaves, NT>>();
     }
     return Kernels();
 }
 
-template <typename T>
+template <typename T, bool NT>
 Kernels tuned(int D, int G, bool append) {
-    if (D == 64) return append ? tuned_g<T, 64, true>(G) : tuned_g<T, 64, false>(G);
-    if (D == 128) return append ? tuned_g<T, 128, true>(G) : tuned_g<T, 128, false>(G);
-    if (D == 256) return append ? tuned_g_few<T, 256, true>(G) : tuned_g_few<T, 256, false>(G);
-    if (D == 96) return append ? tuned_g_few<T, 96, true>(G) : tuned_g_few<T, 96, false>(G);
+    if (D == 64) return append ? tuned_g<T, 64, true, NT>(G) : tuned_g<T, 64, false, NT>(G);
+    if (D == 128) return append ? tuned_g<T, 128, true, NT>(G) : tuned_g<T, 128, false, NT>(G);
+    if (D == 256) return append ? tuned_g_few<T, 256, true, NT>(G) : tuned_g_few<T, 256, false, NT>(G);
+    if (D == 96) return append ? tuned_g_few<T, 96, true, NT>(G) : tuned_g_few<T, 96, false, NT>(G);
     return Kernels();
 }
 

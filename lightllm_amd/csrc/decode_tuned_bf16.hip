@@ -2,5 +2,5 @@
 #include "decode_sched.h"
 
 namespace llkv {
-Kernels tuned_kernels_bf16(int D, int G, bool append) { return tuned<bf16_t>(D, G, append); }
+Kernels tuned_kernels_bf16(int D, int G, bool append) { return tuned<bf16_t, false>(D, G, append); }
 }  // namespace llkv

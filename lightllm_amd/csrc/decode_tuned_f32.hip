@@ -2,5 +2,5 @@
 #include "decode_sched.h"
 
 namespace llkv {
-Kernels tuned_kernels_f32(int D, int G, bool append) { return tuned<float>(D, G, append); }
+Kernels tuned_kernels_f32(int D, int G, bool append) { return tuned<float, false>(D, G, append); }
 }  // namespace llkv

@@ -197,3 +197,84 @@ def test_balanced_merge_entries(long, d, hq, hkv):
         ref = _attend64(q[i:i + 1], k, v, lens[i] - 1)[0]
         bar = 2e-3 * (ref.abs() + ref.square().mean(-1, keepdim=True).sqrt())
         assert torch.all((out[i] - ref).abs() <= bar), (i, float(((out[i] - ref).abs() / bar).max()))
+
+
+# Streaming loads: batches whose bound passes 192 MB.  The bound comes from the table's width, so a
+# wide table gives the large batch's kernels on short sequences (lengths 0, 1, page edges).
+STREAM = [
+    ("f16_balanced", 70, 32, 8, 128, torch.float16, 0, "balanced"),
+    ("bf16_d256_balanced", 40, 16, 8, 256, torch.bfloat16, 0, "balanced"),
+    ("f32_balanced", 200, 14, 2, 64, torch.float32, 0, "balanced"),
+    ("f16_long_chains", 16, 14, 2, 64, torch.float16, 0, "unit"),
+    ("bf16_splits", 12, 32, 32, 96, torch.bfloat16, 4, "splits"),
+    ("f32_one_split", 10, 12, 2, 128, torch.float32, 1, "one_split"),
+]
+
+
+@pytest.mark.parametrize("name,B,hq,hkv,d,dtype,splits,sched", STREAM, ids=[s[0] for s in STREAM])
+def test_decode_streaming_loads(name, B, hq, hkv, d, dtype, splits, sched):
+    g = torch.Generator().manual_seed(len(name))
+    width = max(2048, (250 << 20) // (B * 16 * hkv * d * 2 * dtype.itemsize))
+    bound = width * 16
+    assert kc.decode_schedule(B, hq, hkv, d, bound, dtype, num_splits=splits)[0] == sched
+    lens = torch.randint(1, 700, (B,), generator=g).tolist()
+    lens[:5] = [1, 16, 17, 0, 33]
+    need = [(n + 15) // 16 for n in lens]
+    nb = sum(need) + 1
+    kp = torch.randn(nb, 16, hkv, d, generator=g).to(dtype)
+    vp = torch.randn(nb, 16, hkv, d, generator=g).to(dtype)
+    q, kn, vn = (torch.randn(B, h, d, generator=g).to(dtype) for h in (hq, hkv, hkv))
+    perm = torch.randperm(nb, generator=g).to(torch.int32)
+    table = torch.full((B, width), -1, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = perm[at:at + n]
+        at += n
+    qd, knd, vnd, td = (t.to(DEV) for t in (q, kn, vn, table))
+    ld = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    pools = [(kp.to(DEV), vp.to(DEV)) for _ in range(2)]
+    # append, then decode; the fused call gives the same bits
+    slots = torch.tensor([int(table[i, (n - 1) // 16]) * 16 + (n - 1) % 16 if n else -1 for i, n in enumerate(lens)],
+                         device=DEV)
+    kc.append_kv(knd, vnd, slots, *pools[0])
+    out = kc.paged_decode(qd, *pools[0], td, ld, bound, num_splits=splits)
+    fused = kc.paged_decode_append(qd, knd, vnd, *pools[1], td, ld, bound, num_splits=splits)
+    assert torch.equal(out, fused) and all(torch.equal(a, b) for a, b in zip(*pools))
+    kh, vh = (p.cpu() for p in pools[0])
+    for i in list(range(6)) + [B // 2, B - 1]:
+        if lens[i] == 0:
+            assert torch.all(out[i] == 0)
+            continue
+        rows = table[i, :need[i]].long()
+        k, v = (p[rows].reshape(-1, hkv, d)[:lens[i]] for p in (kh, vh))
+        ref = _attend64(q[i:i + 1], k, v, lens[i] - 1)[0]
+        rms = ref.square().mean(-1, keepdim=True).sqrt()
+        bar = {torch.float32: 1e-6 + 1e-5 * ref.abs(), torch.float16: 2e-3 * (ref.abs() + rms),
+               torch.bfloat16: 1.6e-2 * (ref.abs() + rms)}[dtype]
+        err = (out[i].cpu().double() - ref).abs()
+        assert torch.all(err <= bar), (i, float((err / bar).max()))
+
+
+@pytest.mark.parametrize("extra", [0, 5])
+def test_gather_streaming_edge(extra):
+    """Gathers on both sides of the streaming rule (4 x rows x row bytes at 192 MB), bit for bit."""
+    hkv, d = 8, 128
+    n = (192 << 20) // (4 * hkv * d * 2) + extra
+    g = torch.Generator(device=DEV).manual_seed(5)
+    lens = [n // 3, n - n // 3 - 1, 1]
+    need = [(x + 15) // 16 for x in lens]
+    nb = sum(need) + 2
+    kp = torch.randint(0, 1 << 15, (nb, 16, hkv, d), generator=g, device=DEV, dtype=torch.int16).view(torch.float16)
+    vp = torch.randint(0, 1 << 15, (nb, 16, hkv, d), generator=g, device=DEV, dtype=torch.int16).view(torch.float16)
+    perm = torch.randperm(nb, generator=torch.Generator().manual_seed(6)).to(torch.int32).to(DEV)
+    table = torch.full((3, max(need)), -1, dtype=torch.int32, device=DEV)
+    at, rows = 0, []
+    for i, m in enumerate(need):
+        table[i, :m] = perm[at:at + m]
+        rows.append((perm[at:at + m].long()[:, None] * 16 + torch.arange(16, device=DEV)).reshape(-1)[:lens[i]])
+        at += m
+    cu = torch.tensor([0, lens[0], lens[0] + lens[1], n], dtype=torch.int32, device=DEV)
+    k, v = kc.gather_kv(kp, vp, table, cu, n)
+    rows = torch.cat(rows)
+    for got, pool in ((k, kp), (v, vp)):
+        assert torch.equal(got.view(torch.int16), pool.view(torch.int16).view(-1, hkv, d)[rows])
