@@ -20,15 +20,15 @@
 // Causal masking uses the reference's rule: query i of a P-row chunk over L
 // keys sits at L - P + i and sees keys <= that position.
 //
-// When the units alone would not fill the GPU, key ranges are cut into chunks
-// of chunk_tiles tiles, one work-group each (N x qblocks x max_chunks x Hq
-// work-groups, the q heads of one kv head on one XCD), so that a cached prefix of thousands of keys does not
+// When the units alone would not fill the GPU, key ranges are cut into equal
+// chunks, one work-group each (items x Hq work-groups, the q heads of one kv
+// head on one XCD), so that a cached prefix of thousands of keys does not
 // serialise on one work-group; their partials (normalised fp32 rows + fp32
-// log2-sum-exp2) are merged by
-// prefill_merge_kernel.  The host plans the split from the shape bounds and the
-// kernel's resident work-group count; the kernel then drops it when the units'
-// actual key lengths are even enough (no unit longer than the average load of
-// a compute unit), and the merge kernel follows that decision.
+// log2-sum-exp2) are merged by prefill_merge_kernel.  The host decides from the
+// shape bounds and the kernel's resident work-group count whether a launch may
+// cut; the kernel derives the cuts from the actual key lengths (none when no
+// unit is longer than the average load of a compute unit) and leaves them in a
+// table for the merge kernel.
 #pragma once
 
 #include "attn_common.h"

@@ -129,6 +129,7 @@ constexpr int kMinChunkTiles = 8;
 // 14/2/64 eight 512-row fp16 chunks on prefixes up to 4096: 62.6 us at 10 / 8,
 // 62.3 at 12, 58.6 at 14 and 16; the fp32 form 159 .. 160 at all four.
 constexpr int kShare = 14;
+constexpr int kKeyTiles = (1 << 19) - 1;   // the ranking's key: 19 bits of tiles, 12 of chunks
 
 struct Item {
     int unit, ci, chunks, part;   // part: partial slot of chunk 0 (chunks > 1)
@@ -152,7 +153,7 @@ __device__ inline bool pick_item(const MfmaPrefillArgs& a, int y, int* lds, Item
         return info.tiles >= 0;
     }
     int* tiles = lds;
-    int* key = lds + kRankUnits;   // tiles per chunk << 12 | chunks; -1: no rows
+    int* key = lds + kRankUnits;   // tiles per chunk (at most kKeyTiles) << 12 | chunks; -1: no rows
     int* q0s = lds + 2 * kRankUnits;
     int* ps = lds + 3 * kRankUnits;
     int* ls = lds + 4 * kRankUnits;
@@ -170,7 +171,7 @@ __device__ inline bool pick_item(const MfmaPrefillArgs& a, int y, int* lds, Item
             kvos[u] = r.kvo;
         }
         tiles[u] = r.tiles;
-        key[u] = r.tiles < 0 ? -1 : (r.tiles << 12) | 1;
+        key[u] = r.tiles < 0 ? -1 : (min(r.tiles, kKeyTiles) << 12) | 1;
     }
     if (threadIdx.x == 0) s_item.unit = -1;
     __syncthreads();
@@ -195,7 +196,7 @@ __device__ inline bool pick_item(const MfmaPrefillArgs& a, int y, int* lds, Item
                 const int t = tiles[u];
                 if (t > limit) {
                     const int n = (t + limit - 1) / limit;
-                    key[u] = ((t + n - 1) / n) << 12 | n;
+                    key[u] = min((t + n - 1) / n, kKeyTiles) << 12 | n;
                 }
             }
         }
@@ -224,13 +225,15 @@ __device__ inline bool pick_item(const MfmaPrefillArgs& a, int y, int* lds, Item
         if (cut && blockIdx.x == 0) a.table[u] = make_int2(parts, n);   // for the merge kernel
     }
     __syncthreads();
-    it = s_item;
+    // (the same for every lane: scalar registers)
+    auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    it = Item{uniform(s_item.unit), uniform(s_item.ci), uniform(s_item.chunks), uniform(s_item.part)};
     if (it.unit < 0) return false;
-    info.q0 = q0s[it.unit];
-    info.P = ps[it.unit];
-    info.L = ls[it.unit];
-    info.kvo = kvos[it.unit];
-    info.tiles = tiles[it.unit];
+    info.q0 = uniform(q0s[it.unit]);
+    info.P = uniform(ps[it.unit]);
+    info.L = uniform(ls[it.unit]);
+    info.kvo = uniform(kvos[it.unit]);
+    info.tiles = uniform(tiles[it.unit]);
     return true;
 }
 
