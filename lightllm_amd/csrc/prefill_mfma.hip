@@ -1165,7 +1165,7 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
 // rate, so the number of products decides.
 //
 // Error.  A term pair holds 22 bits, one or two less than fp32; a score's sum
-// takes 3 D / 16 roundings instead of D / 4 and the output's 12 per 64 keys
+// takes 3 D / 16 roundings, D / 16 of them at full size, instead of D / 4 and the output's 12 per 64 keys
 // instead of 16, and those dominate: against 64 bits the result is nearer than
 // the fp32 form's (4.1e-7 there at the shape above).  Below 2^-14 a term is
 // subnormal: with the scales 2^6 (Q, K), 2^8 (V) and 2^7 (P) its rounding is
@@ -1505,20 +1505,38 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
             for (int j = 0; j < CH_T; ++j)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) sq.x[8 * j + e] = vraw[j][e];
+            // The products with a second term first, over every k-step, then x1 y1
+            // (its K terms read again): KS roundings of the sum at its full size.
             uint4 ka[2][2][2];   // [k-step parity][key tile][term]
+            uint4 k1[3][2];      // [k-step mod 3][key tile]: first terms
             auto read_k = [&](int ks, uint4 (&k2)[2][2]) {
 #pragma unroll
                 for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                     for (int p = 0; p < 2; ++p) k2[kt][p] = k_operand(kt, ks, p);
             };
+            auto read_k1 = [&](int ks) {
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt) k1[ks % 3][kt] = k_operand(kt, ks, 0);
+            };
             read_k(0, ka[0]);
             constexpr int M = 6 * KS, M0 = 4;   // MFMAs; those before V's split (its loads have time to land)
             static_for<M>([&](auto kc) {
-                constexpr int k = kc, kt = k & 1, ks = k / 6, pr = (k % 6) / 2;
-                if constexpr (k % 6 == 0 && ks + 1 < KS) read_k(ks + 1, ka[(ks + 1) & 1]);
-                s[kt] = Mfma<_Float16>::mma32(ka[ks & 1][kt][kSplitA[pr]], qop[ks][kSplitB[pr]],
-                                              k < 2 ? f32x16{} : s[kt]);
+                constexpr int k = kc, kt = k & 1;
+                if constexpr (k < 4 * KS) {
+                    constexpr int ks = k / 4, pr = (k % 4) / 2;
+                    if constexpr (k % 4 == 0 && ks + 1 < KS) read_k(ks + 1, ka[(ks + 1) & 1]);
+                    if constexpr (k == 4 * KS - 4) {
+                        read_k1(0);
+                        read_k1(1);
+                    }
+                    s[kt] = Mfma<_Float16>::mma32(ka[ks & 1][kt][kSplitA[pr]], qop[ks][kSplitB[pr]],
+                                                  k < 2 ? f32x16{} : s[kt]);
+                } else {
+                    constexpr int ks = (k - 4 * KS) / 2;
+                    if constexpr (kt == 0 && ks + 2 < KS) read_k1(ks + 2);
+                    s[kt] = Mfma<_Float16>::mma32(k1[ks % 3][kt], qop[ks][0], s[kt]);
+                }
                 if constexpr (k >= M0) {
                     constexpr int s0 = (k - M0) * sq.kSteps / (M - M0), s1 = (k + 1 - M0) * sq.kSteps / (M - M0);
                     static_for<s1 - s0>([&](auto ec) {
