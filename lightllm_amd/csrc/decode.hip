@@ -252,6 +252,11 @@ __global__ __launch_bounds__(1024) void decode_merge_balanced_kernel(DecodeArgs 
 // 14/2/64 fp16 56 -> 53, 61 x 100 .. 2100 of 16/8/256 bf16 106 -> 99); smaller
 // batches may stay cached (64 x 129 .. 2049 of 14/2/64 fp32, 134 MB: 23.6 us, by
 // streaming loads 24.6).
+// Instantiated where it measured faster: the balanced schedule at head_dim 64
+// (93 -> 86 us bf16, 99 -> 90 fp32), 256 (also 144 -> 128 fp32), 128 in 16 bits
+// and 96 in fp32 (183 -> 171), and the 16-wave splits at head_dim 64 in 16 bits.
+// Slower and left plain: fp32 at head_dim 128 (172 -> 194), 16 bits at 96 (252 ->
+// 256), the 16-wave splits at 128 (116 -> 127) and in fp32 (70.5 -> 74.8).
 constexpr int64_t kStreamBytes = 192ll << 20;
 
 // The tuned kernels of a pool type, plain or fused-append (decode_tuned_*.hip).
@@ -543,16 +548,22 @@ int paged_decode_impl(const char* fn, void* out, const void* q, const void* k_ne
                          ((size_t)num_kv_heads * head_dim * es) % 16 == 0;
     Kernels ks;
     if (block_size == kPage && aligned) {
-        const bool stream_kv = (int64_t)num_seqs * max_seq_len * num_kv_heads * head_dim * 2 * (int64_t)es > kStreamBytes;
-        ks = pick_tuned(dtype, head_dim, G, k_new != nullptr, stream_kv);
+        ks = pick_tuned(dtype, head_dim, G, k_new != nullptr);
     }
     const int max_pages_hint = (max_seq_len + block_size - 1) / block_size;
     bool balanced = false, wide = false;
-    // Every call takes the schedule of the plain kernels (from their resident
-    // counts), so that a fused append's results equal append + decode bit for bit
-    // and the loads' form changes no result.
-    const Kernels sched = ks.split != nullptr ? pick_tuned(dtype, head_dim, G, false) : ks;
+    // The fused-append call takes the plain call's schedule (from the plain
+    // kernels' resident counts), so that its results equal append + decode
+    // bit for bit.
+    const Kernels sched = (k_new != nullptr && ks.split != nullptr) ? pick_tuned(dtype, head_dim, G, false) : ks;
     decide_schedule(sched, num_seqs, num_kv_heads, block_size, max_seq_len, num_splits, balanced, wide);
+
+    if (ks.split != nullptr &&
+        (int64_t)num_seqs * max_seq_len * num_kv_heads * head_dim * 2 * (int64_t)es > kStreamBytes) {
+        const Kernels st = pick_tuned(dtype, head_dim, G, k_new != nullptr, true);
+        if (st.balanced != nullptr) ks.balanced = st.balanced;
+        if (st.unit != nullptr) ks.unit = st.unit;
+    }
 
     DecodeArgs a;
     a.out = out;

@@ -165,6 +165,7 @@ struct MfmaDecode {
     static_assert(G >= 1 && G <= 16, "up to 16 query heads per KV head");
     static_assert(D % 32 == 0, "head_dim multiple of 32");
     using T = TT;
+    static constexpr bool kStream = NT;
     using Ops = ScoreOps<T, D>;
     static constexpr int W = WV;              // waves per work-group
     static constexpr int kThreads = 64 * W;

@@ -101,7 +101,7 @@ void decode_balanced_kernel(DecodeArgs a) {
 template <class Body>
 Kernels kernels_of() {
     Kernels k;
-    k.split = decode_split_kernel<Body>;
+    if constexpr (!Body::kStream) k.split = decode_split_kernel<Body>;
     k.balanced = decode_balanced_kernel<Body>;
     return k;
 }
@@ -112,7 +112,8 @@ Kernels kernels_of() {
 template <typename T, int D, int G, bool A, bool NT>
 Kernels kernels_with_unit() {
     Kernels k = kernels_of<MfmaDecode<T, D, G, A, kDecodeWaves, NT>>();
-    if constexpr (!(Elem<T>::kDtype == LLKV_DTYPE_F32 && D == 128))
+    constexpr bool kF32 = Elem<T>::kDtype == LLKV_DTYPE_F32;
+    if constexpr (!(kF32 && D == 128) && (!NT || (D == 64 && !kF32)))
         k.unit = decode_split_kernel<MfmaDecode<T, D, G, A, kUnitWaves, NT>>;
     return k;
 }
@@ -147,12 +148,17 @@ Kernels tuned_g_few(int G) {
     return Kernels();
 }
 
+// NT: the streaming kernels, where they measured faster (kStreamBytes in
+// decode.hip); the others stay null and the plain ones run.
 template <typename T, bool NT>
 Kernels tuned(int D, int G, bool append) {
+    constexpr bool kF32 = Elem<T>::kDtype == LLKV_DTYPE_F32;
     if (D == 64) return append ? tuned_g<T, 64, true, NT>(G) : tuned_g<T, 64, false, NT>(G);
-    if (D == 128) return append ? tuned_g<T, 128, true, NT>(G) : tuned_g<T, 128, false, NT>(G);
+    if constexpr (!NT || !kF32)
+        if (D == 128) return append ? tuned_g<T, 128, true, NT>(G) : tuned_g<T, 128, false, NT>(G);
     if (D == 256) return append ? tuned_g_few<T, 256, true, NT>(G) : tuned_g_few<T, 256, false, NT>(G);
-    if (D == 96) return append ? tuned_g_few<T, 96, true, NT>(G) : tuned_g_few<T, 96, false, NT>(G);
+    if constexpr (!NT || kF32)
+        if (D == 96) return append ? tuned_g_few<T, 96, true, NT>(G) : tuned_g_few<T, 96, false, NT>(G);
     return Kernels();
 }
 
