@@ -1158,7 +1158,7 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
 // instruction's rate (354 us for eight 512-row chunks on prefixes up to 4096,
 // 14/2/64); v_mfma_f32_32x32x16_f16 has 16 times the rate, so the three products
 // cost 0.19 of its matrix time, and the splits are VALU work that runs beside
-// the MFMAs: 158 us there, and 69 -> 37 us for a first prefill of 8 x 77 .. 512
+// the MFMAs: 161 us there, and 69 -> 37 us for a first prefill of 8 x 77 .. 512
 // rows.  Bound now by the latency of a tile's loads and by VALU issue (two
 // waves per SIMD at 256 registers; one at head_dim 96 / 128).  Three bf16 terms (exact) with six products measured 200 us there:
 // with random data the matrix cores sustain about two thirds of their nominal
