@@ -1,6 +1,7 @@
 // MFMA paged prefill attention for gfx950 (fp16 / bf16 here; fp32 pools take
-// kernels of the same schedule, with every operand as two fp16 terms, or at
-// head_dim 256 on 16x16x4 f32; head_dim 64 / 96 / 128 / 256, 16-token pages).  Replaces the reference's scalar prefill kernels
+// kernels of the same schedule, with every operand as three bf16 terms, or at
+// head_dim 256 on 16x16x4 f32; head_dim 64 / 96 / 128 / 256, 16-token pages).
+// Replaces the reference's scalar prefill kernels
 // (src/kv_cache/paged_attention.cu:641-974) for these shapes.
 //
 // Work-group: 4 waves, 128 query rows of one q_head (32 per wave), keys in

@@ -28,10 +28,6 @@ template <> struct Mfma<_Float16> {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
-    __device__ static inline f32x16 mma32(const uint4& a, const uint4& b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
-                                                      __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    }
     __device__ static inline uint32_t pack2(float x, float y) { return pack_h2(x, y); }
     static constexpr uint32_t kOnes = 0x3C003C00u;   // two halves of 1.0
 };
@@ -41,6 +37,10 @@ template <> struct Mfma<bf16_t> {
     __device__ static inline f32x4 mma(const uint4& a, const uint4& b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                       __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    }
+    __device__ static inline f32x16 mma32(const uint4& a, const uint4& b, f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                       __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
     __device__ static inline uint32_t pack2(float x, float y) { return pack_b2(x, y); }
     static constexpr uint32_t kOnes = 0x3F803F80u;   // two bfloat16 1.0
@@ -1149,55 +1149,63 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
     }
 }
 
-// fp32 pools at head_dim 64 / 96 / 128: both products on the fp16 matrix
-// instructions, every operand, scaled by a power of two, as the sum of two fp16
-// terms x = x1 + x2 (x1 = fp16(x), x2 = fp16(x - x1)), and three of the four
-// partial products,
-//     x y = x2 y1 + x1 y2 + x1 y1    (x2 y2 <= 2^-22 |x y| is dropped),
-// summed in fp32.  The fp32 form on v_mfma_f32_16x16x4_f32 ran at 61 % of that
-// instruction's rate (354 us for eight 512-row chunks on prefixes up to 4096,
-// 14/2/64); v_mfma_f32_32x32x16_f16 has 16 times the rate, so the three products
-// cost 0.19 of its matrix time, and the splits are VALU work that runs beside
-// the MFMAs: 161 us there, and 69 -> 37 us for a first prefill of 8 x 77 .. 512
-// rows.  Bound now by the latency of a tile's loads and by VALU issue (two
-// waves per SIMD at 256 registers; one at head_dim 96 / 128).  Three bf16 terms (exact) with six products measured 200 us there:
-// with random data the matrix cores sustain about two thirds of their nominal
-// rate, so the number of products decides.
+// fp32 pools at head_dim 64 / 96 / 128: both products on the bf16 matrix
+// instructions, every operand as the sum of three bf16 terms x = x1 + x2 + x3
+// (x1 = bf16(x), x2 = bf16(x - x1), x3 = x - x1 - x2: 24 bits, what fp32 holds),
+// and six of the nine partial products,
+//     x y = x3 y1 + x2 y2 + x2 y1 + x1 y3 + x1 y2 + x1 y1
+// (x3 y2 + x2 y3 + x3 y3 is below 2^-22 |x y|, 2^-25 on average), summed in fp32.
+// The fp32 form on v_mfma_f32_16x16x4_f32 ran at 61 % of that instruction's rate
+// (356 us for eight 512-row chunks on prefixes up to 4096, 14/2/64);
+// v_mfma_f32_32x32x16_bf16 has 16 times the rate, so the six products cost 0.38
+// of its matrix time, and the splits are VALU work that runs beside the MFMAs:
+// 218 us there, 313 -> 155 us for 32/8/128 chunks of 512, 300 and 77 rows on
+// 1000, 0 and 2000.  Bound by the matrix rate on real data and by VALU issue (two
+// waves per SIMD at 256 registers; one at head_dim 96 / 128; Q's third terms are
+// read from LDS: 222 -> 218 and 176 -> 155 us).
+// Two fp16 terms and three products take 172 and 120 us, but hold 22 bits, and
+// fewer below 2^-14 of a scale: a V channel of 1e-6 beside channels of one came
+// out 7e-5 off, prompts of five rows 9.2e-8 (this form 5.5e-8, the fp32 form
+// 7.1e-8), and finite V of 1e34 overflowed their scales.
 //
-// Error.  A term pair holds 22 bits, one or two less than fp32; a score's sum
-// takes 3 D / 16 roundings, D / 16 of them at full size, instead of D / 4 and the output's 12 per 64 keys
-// instead of 16, and those dominate: against 64 bits the result is nearer than
-// the fp32 form's (4.1e-7 there at the shape above).  Below 2^-14 a term is
-// subnormal: with the scales 2^6 (Q, K), 2^8 (V) and 2^7 (P) its rounding is
-// <= 2^-31 absolute, so a tile counts as fit when its largest magnitude is in
-// [2^-8, 2^9] (2^-10, 2^7 for V) or zero, and the rounding is then <= 2^-23 of
-// that magnitude.  A tile or a Q that is not fit (infinities included) runs on
-// the fp32 matrix instructions: it is staged again as plain fp32, high halves in
-// the first plane and low halves in the second.
+// Error.  A score sums its products with a second or third term first, over every
+// k-step, then x1 y1 (D / 16 roundings at its full size; the fp32 form D / 4).  The
+// output and the row sums take a tile's sum in one addition, where the fp32 form
+// rounds them 16 times per 64 keys: 5.0e-7 -> 3.0e-7 against 64 bits for 512 rows
+// on 4096, 14/2/64, and with the output's products summed in place 5.2e-7 (215 us).
 //
-// K and V tiles lie in LDS as two planes with the operand layout of the 16-bit
+// bf16 has the exponents of fp32, so nothing is scaled.  A tile or a Q whose
+// largest magnitude is beyond 2^60 (infinities included) or, not being zero, below
+// 2^-60 runs on the fp32 matrix instructions: within these bounds no sum of
+// products of terms overflows.  In a tile that has larger values, one below 2^-110
+// keeps an absolute error of at most 2^-126, the smallest normal number.  A tile
+// that does not fit is staged again as plain fp32, high halves in the first plane
+// and low halves in the second.
+//
+// K and V tiles lie in LDS as three planes with the operand layout of the 16-bit
 // kernel (V^T by transposing reads), split once per work-group while staging.
-constexpr float kScaleQK = 64.0f, kScaleV = 256.0f, kShiftP = 7.0f;   // P: 2^7
-constexpr float kFitMax = 32768.0f, kFitMin = 0.25f;                  // scaled magnitudes
+constexpr int kTerms = 3, kProducts = 6;
+constexpr float kFitMax = 0x1p60f, kFitMin = 0x1p-60f;
 
-// x - float(low / high half of w): one v_fma_mix_f32 each.
-__device__ inline float minus_lo(float x, uint32_t w) {
-    return __builtin_fmaf((float)__builtin_bit_cast(half2_v, w).x, -1.0f, x);
-}
-__device__ inline float minus_hi(float x, uint32_t w) {
-    return __builtin_fmaf((float)__builtin_bit_cast(half2_v, w).y, -1.0f, x);
-}
+// x - float(low / high half of w).
+__device__ inline float minus_lo(float x, uint32_t w) { return x - __uint_as_float(w << 16); }
+__device__ inline float minus_hi(float x, uint32_t w) { return x - __uint_as_float(w & 0xFFFF0000u); }
 
-// The two fp16 terms of 8 values, two per word.
-__device__ inline void split8(const float (&x)[8], uint4 (&t)[2]) {
-    uint32_t w[2][4];
+// The three bf16 terms of 8 values, two per word.
+__device__ inline void split8(const float (&x)[8], uint4 (&t)[kTerms]) {
+    uint32_t w[kTerms][4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        w[0][j] = pack_h2(x[2 * j], x[2 * j + 1]);
-        w[1][j] = pack_h2(minus_lo(x[2 * j], w[0][j]), minus_hi(x[2 * j + 1], w[0][j]));
+        float a = x[2 * j], b = x[2 * j + 1];
+#pragma unroll
+        for (int p = 0; p < kTerms; ++p) {
+            w[p][j] = pack_b2(a, b);
+            a = minus_lo(a, w[p][j]);
+            b = minus_hi(b, w[p][j]);
+        }
     }
 #pragma unroll
-    for (int p = 0; p < 2; ++p) t[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+    for (int p = 0; p < kTerms; ++p) t[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
 }
 
 // 8 plain fp32 values in the same place, and element e of them.
@@ -1219,7 +1227,7 @@ __device__ inline float plain(const uint4 (&t)[2], int e) {
 }
 
 // Uniform over the wave: the largest magnitudes `most` of its lanes do not fit
-// the two terms.  (A NaN passes as one: it stays NaN in either form.)
+// the terms.  (A NaN passes as one: it stays NaN in either form.)
 __device__ inline bool unfit(float most) {
     return __builtin_amdgcn_ballot_w64(most > kFitMax) != 0 ||
            (__builtin_amdgcn_ballot_w64(most >= kFitMin) == 0 && __builtin_amdgcn_ballot_w64(most > 0.0f) != 0);
@@ -1235,35 +1243,60 @@ __device__ inline void static_for(F f) {
     static_for_impl(f, std::make_integer_sequence<int, N>());
 }
 
-// The three products in the order of accumulation: term of A, term of B.
-constexpr int kSplitA[3] = {1, 0, 0};
-constexpr int kSplitB[3] = {0, 1, 0};
+// The six products in the order of accumulation: term of A, term of B.
+constexpr int kProdA[kProducts] = {2, 1, 1, 0, 0, 0};
+constexpr int kProdB[kProducts] = {0, 1, 0, 2, 1, 0};
 
-// split8 of 2 N values times `scale` in 2 N steps of three VALU instructions or
-// so, to be issued one by one between MFMAs: a 32x32x16 MFMA holds the matrix
-// core for 32 cycles, in which a wave can issue VALU instructions, but only
-// those that stand between it and the next MFMA (issue is in order, and the
-// compiler by itself puts all VALU work of a region on one side of its MFMAs).
+// Order of a score's products over K k-steps: per k-step the first five, then,
+// again per k-step, x1 y1.  Their A operands come in 4 K groups (one term of one
+// k-step), read kAhead groups before their first product into a ring of kAhead + 1.
+template <int K>
+struct ScoreChain {
+    static constexpr int kLength = kProducts * K, kGroups = 4 * K;
+    static constexpr bool small(int i) { return i < 5 * K; }
+    static constexpr int step(int i) { return small(i) ? i / 5 : i - 5 * K; }        // k-step of product i
+    static constexpr int prod(int i) { return small(i) ? i % 5 : kProducts - 1; }
+    static constexpr int group(int i) { return small(i) ? 3 * step(i) + 2 - kProdA[prod(i)] : 3 * K + step(i); }
+    static constexpr bool first(int i) { return i == 0 || group(i) != group(i - 1); }
+    static constexpr int group_step(int g) { return g < 3 * K ? g / 3 : g - 3 * K; }
+    static constexpr int group_term(int g) { return g < 3 * K ? 2 - g % 3 : 0; }
+};
+
+// split8 of 2 N values in 4 N steps of three VALU instructions or so, to be
+// issued one by one between MFMAs: a 32x32x16 MFMA holds the matrix core for 32
+// cycles, in which a wave can issue VALU instructions, but only those that stand
+// between it and the next MFMA (issue is in order, and the compiler by itself
+// puts all VALU work of a region on one side of its MFMAs).
 template <int N>
 struct SplitSeq {
-    static constexpr int kSteps = 2 * N;
+    static constexpr int kSteps = 4 * N, kStepsOf8 = 16;
     float x[2 * N];
-    uint32_t w[2][N];
-    float most;   // largest scaled magnitude (step 0 starts it)
+    uint32_t w[kTerms][N];
+    float most;   // largest magnitude (step 0 starts it)
     template <bool FIT>
-    __device__ void step(int i, float scale) {
-        const int j = i >> 1;
+    __device__ void step(int i) {
+        const int j = i >> 2;
         float &a = x[2 * j], &b = x[2 * j + 1];
-        if ((i & 1) == 0) {
-            if constexpr (FIT) {
-                a *= scale;
-                b *= scale;
-                const float ab = fmaxf(fabsf(a), fabsf(b));
-                most = i == 0 ? ab : fmaxf(most, ab);
-            }
-            w[0][j] = pack_h2(a, b);
-        } else {
-            w[1][j] = pack_h2(minus_lo(a, w[0][j]), minus_hi(b, w[0][j]));
+        switch (i & 3) {
+            case 0:
+                if constexpr (FIT) {
+                    const float ab = fmaxf(fabsf(a), fabsf(b));
+                    most = i == 0 ? ab : fmaxf(most, ab);
+                }
+                w[0][j] = pack_b2(a, b);
+                break;
+            case 1:
+                a = minus_lo(a, w[0][j]);
+                b = minus_hi(b, w[0][j]);
+                break;
+            case 2:
+                w[1][j] = pack_b2(a, b);
+                a = minus_lo(a, w[1][j]);
+                break;
+            case 3:
+                b = minus_hi(b, w[1][j]);
+                w[2][j] = pack_b2(a, b);
+                break;
         }
     }
     __device__ uint4 term(int p, int c) const {   // values 8 c .. 8 c + 7
@@ -1277,13 +1310,14 @@ struct SmemSplit {
     static constexpr int PAD = kSwz ? D : D + 8;          // halves per row
     union {
         struct {
-            alignas(16) uint16_t k[2][BN * PAD];
-            alignas(16) uint16_t v[2][BN * PAD];
+            alignas(16) uint16_t k[kTerms][BN * PAD];
+            alignas(16) uint16_t v[kTerms][BN * PAD];
         };
         int order[6 * kRankUnits];
     };
+    alignas(16) uint4 q3[4][D / 16][64];   // third terms of Q: [wave][k-step][lane]
     int pages[kPageWindow];
-    int plain[2][2];   // [K, V][tile parity]: the latest such tile that does not fit two terms
+    int plain[2][2];   // [K, V][tile parity]: the latest such tile that does not fit the terms
     int plain_q;       // a wave's Q does not fit
 };
 
@@ -1319,7 +1353,7 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
 
     // Q^T operands: lane (h, c32) holds dims 16 ks + 8 h .. + 7 of query c32.
     const int ql = q_lo + w * WQ + c32;
-    uint4 qop[KS][2];
+    uint4 qop[KS][2];   // first and second terms (the third: sm.q3)
     const float* qrow = reinterpret_cast<const float*>(a.q) + ((int64_t)(q0 + ql) * a.Hq + hq) * D + h * 8;
     auto read_q = [&](int ks, float (&x)[8]) {
 #pragma unroll
@@ -1338,11 +1372,12 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
             float x[8];
             read_q(ks, x);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                x[e] *= kScaleQK;
-                most = fmaxf(most, fabsf(x[e]));
-            }
-            split8(x, qop[ks]);
+            for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(x[e]));
+            uint4 tm[kTerms];
+            split8(x, tm);
+            qop[ks][0] = tm[0];
+            qop[ks][1] = tm[1];
+            sm.q3[w][ks][lane] = tm[2];
         }
         if (unfit(most) && lane == 0) sm.plain_q = 1;
     };
@@ -1408,27 +1443,24 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
             for (int e = 0; e < 4; ++e) raw[j][e] = lo[e], raw[j][4 + e] = hi[e];
         }
     };
-    // Splits a staged tile into its planes; returns the lane's largest scaled magnitude.
-    auto split_tile = [&](float (&raw)[CH_T][8], uint16_t (&planes)[2][BN * PAD], const int (&dst)[CH_T],
-                          float scale) {
+    // Splits a staged tile into its planes; returns the lane's largest magnitude.
+    auto split_tile = [&](const float (&raw)[CH_T][8], uint16_t (&planes)[kTerms][BN * PAD],
+                          const int (&dst)[CH_T]) {
         float most = 0.0f;
 #pragma unroll
         for (int j = 0; j < CH_T; ++j) {
-            uint4 tm[2];
+            uint4 tm[kTerms];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                raw[j][e] *= scale;
-                most = fmaxf(most, fabsf(raw[j][e]));
-            }
+            for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(raw[j][e]));
             split8(raw[j], tm);
 #pragma unroll
-            for (int p = 0; p < 2; ++p) *reinterpret_cast<uint4*>(&planes[p][dst[j]]) = tm[p];
+            for (int p = 0; p < kTerms; ++p) *reinterpret_cast<uint4*>(&planes[p][dst[j]]) = tm[p];
         }
         return most;
     };
     // After a split that found tile t of K (kv 0) or V (kv 1) unfit: the whole
     // tile once more, plain.  Called by every wave (it ends with a barrier).
-    auto restage_plain = [&](uint16_t (&planes)[2][BN * PAD], const int (&dst)[CH_T], const char* base, int t) {
+    auto restage_plain = [&](uint16_t (&planes)[kTerms][BN * PAD], const int (&dst)[CH_T], const char* base, int t) {
         float raw[CH_T][8];
         load_tile(base, t, raw);
 #pragma unroll
@@ -1456,26 +1488,23 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
     };
     // A operand of O^T: lane holds dim 32 dt + c32 of keys 16 j + 8 h .. + 7
     // (transposing reads, as in the 16-bit kernel).
-    auto v_operand = [&](int dt, int j, uint4 (&va)[2]) {
+    auto v_operand = [&](int dt, int j, int p) {
         typedef short s16x4 __attribute__((ext_vector_type(4)));
         typedef unsigned u32x2v __attribute__((ext_vector_type(2)));
         const int r0 = 16 * j + 8 * h + ((lane & 15) >> 2), hc = dt * 32 + (lane & 16) + 4 * (lane & 3);
         const int a0 = r0 * PAD + vcol(r0, hc), a1 = (r0 + 4) * PAD + vcol(r0 + 4, hc);
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const u32x2v lo = __builtin_bit_cast(u32x2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4*)(&sm.v[p][a0])));
-            const u32x2v hi = __builtin_bit_cast(u32x2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4*)(&sm.v[p][a1])));
-            va[p] = make_uint4(lo.x, lo.y, hi.x, hi.y);
-        }
+        const u32x2v lo = __builtin_bit_cast(u32x2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(&sm.v[p][a0])));
+        const u32x2v hi = __builtin_bit_cast(u32x2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(&sm.v[p][a1])));
+        return make_uint4(lo.x, lo.y, hi.x, hi.y);
     };
     if (t_begin < t_end) {
         stage_pages(4 * t_begin);
         load_tile(kb_, t_begin, kraw);
         load_tile(vb_, t_begin, vraw);
         load_q();
-        if (unfit(split_tile(kraw, sm.k, kdst, kScaleQK)) && lane == 0) sm.plain[0][t_begin & 1] = t_begin;
+        if (unfit(split_tile(kraw, sm.k, kdst)) && lane == 0) sm.plain[0][t_begin & 1] = t_begin;
     }
     lds_barrier();
 
@@ -1497,55 +1526,40 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
         // ---- S^T = K Q^T; the lane's scores are keys 32 kt + 16 (i / 8) + 8 h + i % 8
         f32x16 s[2];
         float v_most, k_most;
-        float c = a.scale_log2;
+        const float c = a.scale_log2;
         if (__builtin_expect(!k_plain, 1)) {
-            c *= 1.0f / (kScaleQK * kScaleQK);
             SplitSeq<4 * CH_T> sq;
 #pragma unroll
             for (int j = 0; j < CH_T; ++j)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) sq.x[8 * j + e] = vraw[j][e];
-            // The products with a second term first, over every k-step, then x1 y1
-            // (its K terms read again): KS roundings of the sum at its full size.
-            uint4 ka[2][2][2];   // [k-step parity][key tile][term]
-            uint4 k1[3][2];      // [k-step mod 3][key tile]: first terms
-            auto read_k = [&](int ks, uint4 (&k2)[2][2]) {
+            typedef ScoreChain<KS> Ch;
+            constexpr int kAhead = 2;
+            uint4 ka[kAhead + 1][2];   // [group][key tile]
+            uint4 q3;
+            auto read_k = [&](int gr) {
 #pragma unroll
                 for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int p = 0; p < 2; ++p) k2[kt][p] = k_operand(kt, ks, p);
+                    ka[gr % (kAhead + 1)][kt] = k_operand(kt, Ch::group_step(gr), Ch::group_term(gr));
             };
-            auto read_k1 = [&](int ks) {
 #pragma unroll
-                for (int kt = 0; kt < 2; ++kt) k1[ks % 3][kt] = k_operand(kt, ks, 0);
-            };
-            read_k(0, ka[0]);
-            constexpr int M = 6 * KS, M0 = 4;   // MFMAs; those before V's split (its loads have time to land)
+            for (int gr = 0; gr < kAhead; ++gr) read_k(gr);
+            constexpr int M = 2 * Ch::kLength, M0 = 4;   // MFMAs; those before V's split (its loads have time to land)
             static_for<M>([&](auto kc) {
-                constexpr int k = kc, kt = k & 1;
-                if constexpr (k < 4 * KS) {
-                    constexpr int ks = k / 4, pr = (k % 4) / 2;
-                    if constexpr (k % 4 == 0 && ks + 1 < KS) read_k(ks + 1, ka[(ks + 1) & 1]);
-                    if constexpr (k == 4 * KS - 4) {
-                        read_k1(0);
-                        read_k1(1);
-                    }
-                    s[kt] = Mfma<_Float16>::mma32(ka[ks & 1][kt][kSplitA[pr]], qop[ks][kSplitB[pr]],
-                                                  k < 2 ? f32x16{} : s[kt]);
-                } else {
-                    constexpr int ks = (k - 4 * KS) / 2;
-                    if constexpr (kt == 0 && ks + 2 < KS) read_k1(ks + 2);
-                    s[kt] = Mfma<_Float16>::mma32(k1[ks % 3][kt], qop[ks][0], s[kt]);
-                }
+                constexpr int k = kc, i = k / 2, kt = k & 1, ks = Ch::step(i), gr = Ch::group(i), qt = kProdB[Ch::prod(i)];
+                if constexpr (kt == 0 && Ch::first(i) && gr + kAhead < Ch::kGroups) read_k(gr + kAhead);
+                if constexpr (kt == 0 && i < 5 * KS && i % 5 == 0) q3 = sm.q3[w][ks][lane];
+                s[kt] = Mfma<bf16_t>::mma32(ka[gr % (kAhead + 1)][kt], qt == 2 ? q3 : qop[ks][qt & 1],
+                                            i == 0 ? f32x16{} : s[kt]);
                 if constexpr (k >= M0) {
                     constexpr int s0 = (k - M0) * sq.kSteps / (M - M0), s1 = (k + 1 - M0) * sq.kSteps / (M - M0);
                     static_for<s1 - s0>([&](auto ec) {
                         constexpr int st = s0 + ec;
-                        sq.template step<true>(st, kScaleV);
-                        if constexpr (st % 8 == 7) {
+                        sq.template step<true>(st);
+                        if constexpr ((st + 1) % sq.kStepsOf8 == 0) {
 #pragma unroll
-                            for (int p = 0; p < 2; ++p)
-                                *reinterpret_cast<uint4*>(&sm.v[p][vdst[st / 8]]) = sq.term(p, st / 8);
+                            for (int p = 0; p < kTerms; ++p)
+                                *reinterpret_cast<uint4*>(&sm.v[p][vdst[st / sq.kStepsOf8]]) = sq.term(p, st / sq.kStepsOf8);
                         }
                     });
                 }
@@ -1567,7 +1581,7 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
                         s[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(plain(ka, e), x[e], s[kt], 0, 0, 0);
                 }
             }
-            v_most = split_tile(vraw, sm.v, vdst, kScaleV);
+            v_most = split_tile(vraw, sm.v, vdst);
         }
         if (unfit(v_most) && lane == 0) sm.plain[1][t & 1] = t;
         lds_barrier();   // V of the tile is in LDS; every wave is done with the K buffer
@@ -1601,54 +1615,65 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
             for (int dt = 0; dt < DT; ++dt) o[dt] *= corr;
         }
 
-        // ---- P = 2^(S c - m + 7), O^T += V^T P^T, one 16-key step at a time --
-        const float mp = m - kShiftP;
+        // ---- P = 2^(S c - m), O^T += V^T P^T ------------------------------
         if (__builtin_expect(!v_plain, 1)) {
-            uint4 pop[2];
+            // P's terms of 16-key step j + 1 are made beside the MFMAs of step j, the
+            // next tile's K is split beside the last step's (after the last tile: into a
+            // buffer nobody reads).
+            uint4 pop[kTerms];
+            float psum = 0.0f;
             {
                 float p[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    p[e] = fast_exp2(fmaf(s[0][e], c, -mp));
-                    lsum += p[e];
+                    p[e] = fast_exp2(fmaf(s[0][e], c, -m));
+                    psum += p[e];
                 }
                 split8(p, pop);
             }
-            SplitSeq<4 * CH_T> sq;   // the next tile's K (after the last tile: into a buffer nobody reads)
+            SplitSeq<4 * CH_T> sq;
 #pragma unroll
             for (int j = 0; j < CH_T; ++j)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) sq.x[8 * j + e] = kraw[j][e];
-            static_for<4>([&](auto jc) {
-                constexpr int j = jc, M = 3 * DT;   // MFMAs of the step
-                uint4 va[DT][2];
+            constexpr int kGroups = 4 * kTerms;
+            uint4 va[2][DT];   // [group (a term of a step) mod 2]
+            auto read_v = [&](int gr) {
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) v_operand(dt, j, va[dt]);
-                SplitSeq<4> ps;   // the next step's probabilities
+                for (int dt = 0; dt < DT; ++dt) va[gr & 1][dt] = v_operand(dt, gr / kTerms, 2 - gr % kTerms);
+            };
+            read_v(0);
+            f32x16 od[DT];   // the tile's sums
+            static_for<4>([&](auto jc) {
+                constexpr int j = jc, M = kProducts * DT;
+                SplitSeq<4> ps;
                 static_for<M>([&](auto kc) {
-                    constexpr int k = kc, dt = k % DT, pr = k / DT;
-                    o[dt] = Mfma<_Float16>::mma32(va[dt][kSplitA[pr]], pop[kSplitB[pr]], o[dt]);
+                    constexpr int k = kc, dt = k % DT, pr = k / DT, gr = kTerms * j + 2 - kProdA[pr];
+                    constexpr bool first = pr == 0 || kProdA[pr] != kProdA[pr - (pr > 0)];   // of its group
+                    if constexpr (dt == 0 && first && gr + 1 < kGroups) read_v(gr + 1);
+                    od[dt] = Mfma<bf16_t>::mma32(va[gr & 1][dt], pop[kProdB[pr]],
+                                                 j == 0 && pr == 0 ? f32x16{} : od[dt]);
                     if constexpr (j < 3) {   // 8 exponentials, then their terms
-                        constexpr int s0 = k * 16 / M, s1 = (k + 1) * 16 / M;
+                        constexpr int s0 = k * (8 + ps.kSteps) / M, s1 = (k + 1) * (8 + ps.kSteps) / M;
                         static_for<s1 - s0>([&](auto ec) {
                             constexpr int st = s0 + ec;
                             if constexpr (st < 8) {
                                 constexpr int e = 8 * (j + 1) + st;
-                                ps.x[st] = fast_exp2(fmaf(s[e >> 4][e & 15], c, -mp));
-                                lsum += ps.x[st];
+                                ps.x[st] = fast_exp2(fmaf(s[e >> 4][e & 15], c, -m));
+                                psum += ps.x[st];
                             } else {
-                                ps.template step<false>(st - 8, 1.0f);
+                                ps.template step<false>(st - 8);
                             }
                         });
                     } else {
                         constexpr int s0 = k * sq.kSteps / M, s1 = (k + 1) * sq.kSteps / M;
                         static_for<s1 - s0>([&](auto ec) {
                             constexpr int st = s0 + ec;
-                            sq.template step<true>(st, kScaleQK);
-                            if constexpr (st % 8 == 7) {
+                            sq.template step<true>(st);
+                            if constexpr ((st + 1) % sq.kStepsOf8 == 0) {
 #pragma unroll
-                                for (int p = 0; p < 2; ++p)
-                                    *reinterpret_cast<uint4*>(&sm.k[p][kdst[st / 8]]) = sq.term(p, st / 8);
+                                for (int p = 0; p < kTerms; ++p)
+                                    *reinterpret_cast<uint4*>(&sm.k[p][kdst[st / sq.kStepsOf8]]) = sq.term(p, st / sq.kStepsOf8);
                             }
                         });
                     }
@@ -1656,34 +1681,37 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
                 });
                 if constexpr (j < 3) {
 #pragma unroll
-                    for (int p = 0; p < 2; ++p) pop[p] = ps.term(p, 0);
+                    for (int p = 0; p < kTerms; ++p) pop[p] = ps.term(p, 0);
                 }
             });
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) o[dt] += od[dt];
+            lsum += psum;
             k_most = sq.most;
         } else {
             // (an opaque copy: the exponentials of the two branches must not be
             // merged and moved ahead of the branch)
-            float mq = mp;
+            float mq = m;
             asm volatile("" : "+v"(mq));
+            float psum = 0.0f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 float p[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     p[e] = fast_exp2(fmaf(s[j >> 1][8 * (j & 1) + e], c, -mq));
-                    lsum += p[e];
-                    p[e] *= kScaleV;   // (V is plain here, scaled in the other tiles)
+                    psum += p[e];
                 }
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) {
-                    uint4 va[2];
-                    v_operand(dt, j, va);
+                    const uint4 va[2] = {v_operand(dt, j, 0), v_operand(dt, j, 1)};
 #pragma unroll
                     for (int e = 0; e < 8; ++e)   // contracts keys 16 j + 8 h + e
                         o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(plain(va, e), p[e], o[dt], 0, 0, 0);
                 }
             }
-            k_most = split_tile(kraw, sm.k, kdst, kScaleQK);
+            lsum += psum;
+            k_most = split_tile(kraw, sm.k, kdst);
         }
         if (unfit(k_most) && lane == 0) sm.plain[0][(t + 1) & 1] = t + 1;
         lds_barrier();   // K of the next tile is in LDS; every wave is done with the V buffer
@@ -1691,7 +1719,7 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
 
     lsum += __shfl_xor(lsum, 32, 64);
     if (ql >= P) return;
-    const float inv = lsum > 0.f ? 1.0f / (kScaleV * lsum) : 0.f;
+    const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
     const int64_t prow = ((int64_t)wk.part * a.Hq + hq) * BQ + w * WQ + c32;
     float* drow = wk.direct ? reinterpret_cast<float*>(a.out) + ((int64_t)(q0 + ql) * a.Hq + hq) * D
                             : a.part_o + prow * D;
@@ -1701,7 +1729,7 @@ void prefill_f32_split_kernel(MfmaPrefillArgs a) {
         for (int i = 0; i < 4; ++i)
             *reinterpret_cast<float4*>(drow + dt * 32 + 8 * i + 4 * h) =
                 make_float4(o[dt][4 * i] * inv, o[dt][4 * i + 1] * inv, o[dt][4 * i + 2] * inv, o[dt][4 * i + 3] * inv);
-    if (!wk.direct && h == 0) a.part_lse[prow] = lsum > 0.f ? m - kShiftP + fast_log2(lsum) : -INFINITY;
+    if (!wk.direct && h == 0) a.part_lse[prow] = lsum > 0.f ? m + fast_log2(lsum) : -INFINITY;
 }
 
 // Four consecutive output elements from fp32 values.

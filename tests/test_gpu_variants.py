@@ -49,9 +49,8 @@ def _attend64(q, k, v, hist):
     return torch.einsum("hpl,lhd->phd", torch.softmax(s, -1), vv)
 
 
-# fp32 prefill by two fp16 terms (head_dim 64, 96, 128): tile remainders, and tiles that do not fit
-# the two terms (they run on the fp32 matrix instructions), at the edges of the rule: one value
-# beyond 2^9, infinities, whole tensors too small, q too large.
+# fp32 prefill by terms (head_dim 64, 96, 128): tile remainders, large and small values and
+# infinities, mostly in launches that cut nothing (test_prefill_f32_terms_cut has the cuts).
 SPLIT = ["plain", "k_one_large", "k_minus_inf", "v_one_inf", "v_tiny", "k_tiny_q_large", "k_large_window",
          "v_zero"]
 
@@ -114,6 +113,109 @@ def test_prefill_f32_split_terms(case, d):
         assert torch.equal(out[~fine], ref[~fine]), (case, name)
         err = (out - ref)[fine].abs()
         assert torch.all(err <= 1e-6 * unit + 1e-5 * ref[fine].abs()), (case, name, float(err.max()))
+
+
+# The same with cut key ranges (35 tiles in chunks of 7), with values on both sides of what the
+# terms hold (2^-60 .. 2^60; other tiles run on the fp32 matrix instructions) in the first tile of
+# a later chunk (keys 448 ..) and inside one (keys 576 ..), and finite values of any size and of
+# mixed sizes, whose dims are each as exact as dims of one.
+TERMS = ["plain", "k_beyond", "k_minus_inf", "k_tiny_q_large", "v_beyond", "v_edge", "v_1e35", "v_one_inf",
+         "v_tiny", "v_mixed_dims", "v_zero"]
+
+
+@pytest.mark.parametrize("d", [64, 96, 128])
+@pytest.mark.parametrize("case", TERMS)
+def test_prefill_f32_terms_cut(case, d):
+    g = torch.Generator().manual_seed(len(case) + d)
+    hq, hkv, P, L = 4, 2, 133, 2200
+    q = torch.randn(P, hq, d, generator=g)
+    k = torch.randn(L, hkv, d, generator=g)
+    v = torch.randn(L, hkv, d, generator=g)
+    unit = torch.ones(d, dtype=torch.float64)
+    if case == "k_beyond":
+        q[..., 3] *= 1e-20
+        k[450, :, 3] = 3e20
+        k[600, :, 3] = -2e20
+    elif case == "k_minus_inf":     # the keys drop out of the softmax
+        q[..., 5] = q[..., 5].abs() + 0.1
+        k[450, 0, 5] = k[600, 1, 5] = float("-inf")
+    elif case == "k_tiny_q_large":
+        k *= 1e-20
+        q *= 1e20
+    elif case == "v_beyond":
+        v[450:460] *= 1e30
+        v[600] *= 1e30
+        unit *= 1e30
+    elif case == "v_edge":
+        v[450], v[600] = 2.0 ** 60, 2.0 ** 60 * (1 + 2.0 ** -23)
+        unit *= 2.0 ** 60
+    elif case == "v_1e35":
+        v *= 1e35
+        unit *= 1e35
+    elif case == "v_one_inf":       # keys that every row sees
+        v[450, 1, 7] = float("inf")
+        v[600, 0, 9] = float("-inf")
+    elif case == "v_tiny":
+        v *= 1e-25
+        unit *= 1e-25
+    elif case == "v_mixed_dims":
+        unit = 10.0 ** -(torch.arange(d) % 12).double()
+        v *= unit.float()
+    elif case == "v_zero":
+        v.zero_()
+        k[448:512] = 0
+    nb = (L + 15) // 16
+    perm = torch.randperm(nb, generator=g)
+    kp, vp = torch.zeros(nb, 16, hkv, d), torch.zeros(nb, 16, hkv, d)
+    pos = torch.arange(L)
+    kp[perm[pos // 16], pos % 16], vp[perm[pos // 16], pos % 16] = k, v
+    assert kc.lib().llkv_paged_prefill_workspace_size(1, P, P, L, hq, d, 16, kc.dtype_code(q.dtype)) > 0
+    cu, lens = torch.tensor([0, P], dtype=torch.int32, device=DEV), torch.tensor([L], dtype=torch.int32, device=DEV)
+    out = kc.paged_prefill(q.to(DEV), kp.to(DEV), vp.to(DEV), perm.to(torch.int32).reshape(1, -1).to(DEV), cu, lens,
+                           P, L).cpu().double()
+    ref = _attend64(q, k, v, L - P)
+    fine = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(out), fine)
+    assert torch.equal(out[~fine], ref[~fine])
+    bar = 1e-6 * unit + 1e-5 * ref.abs()
+    assert torch.all(((out - ref).abs() <= bar)[fine]), float(((out - ref).abs() / bar)[fine].max())
+
+
+# 2-norm errors against 64 bits: 1e-6 is 17 roundings of 2^-24; the row sum and the output take one
+# per 64-key tile (24 tiles), at random sizes and signs, and the fp32 matrix instructions' own
+# summation is 5e-7 off.  Dims of 1e-4 .. 1e-10 beside dims of one, K with a constant large dim (scores
+# of 112, of which 2^-24 is 7e-6), a few rows.
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (4, 4, 96), (8, 2, 128)])
+def test_prefill_f32_holds_32_bits(hq, hkv, d):
+    def run(P, L, change, dims=slice(None)):
+        g = torch.Generator().manual_seed(P + L)
+        q, k, v = (torch.randn(n, h, d, generator=g) for n, h in ((P, hq), (L, hkv), (L, hkv)))
+        change(q, k, v)
+        nb = (L + 15) // 16
+        kp, vp = torch.zeros(nb * 16, hkv, d), torch.zeros(nb * 16, hkv, d)
+        kp[:L], vp[:L] = k, v
+        ids = torch.arange(nb, dtype=torch.int32).reshape(1, -1)
+        out = kc.paged_prefill(q.to(DEV), kp.view(nb, 16, hkv, d).to(DEV), vp.view(nb, 16, hkv, d).to(DEV), ids.to(DEV),
+                               torch.tensor([0, P], dtype=torch.int32, device=DEV),
+                               torch.tensor([L], dtype=torch.int32, device=DEV), P, L).cpu().double()[..., dims]
+        ref = _attend64(q, k, v, L - P)[..., dims]
+        return float(torch.linalg.vector_norm(out - ref) / torch.linalg.vector_norm(ref))
+
+    def dim7(scale):
+        def change(q, k, v):
+            v[..., 7] *= scale
+        return change
+
+    def biased(q, k, v):
+        k[..., 3] += 300 * d ** 0.5 / 8
+        q[..., 3] = 3
+
+    for scale in (1.0, 1e-4, 1e-6, 1e-10):
+        assert run(150, 1500, dim7(scale), dims=7) <= 1e-6, scale
+    # five rows on nothing: at most five keys, so the roundings are those of a score (D / 16 at its
+    # full size, 2^-24 each at random) and of single products: the fp32 instructions give 7.1e-8 .. 8.1e-8
+    assert run(5, 5, dim7(1.0)) <= 8.1e-8
+    assert run(150, 1500, biased) <= 3e-5
 
 
 # Work items of a prefill launch: (prefixes, chunks) with cut key ranges (one long sequence: many
