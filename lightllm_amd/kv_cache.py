@@ -33,7 +33,8 @@ def dtype_code(t: torch.dtype) -> int:
 
 # The smallest calls are bound by the host, so a call passes addresses as plain
 # integers (the argument types of _lib.py convert them) and asks for the raw
-# current stream: a one-sequence append + decode 15.2 -> 11.4 us a call.
+# current stream: a one-sequence append + decode 15.0 -> 10.3 .. 12.0 us a call, also with
+# max_seq_len growing by one from call to call.
 def _ptr(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
@@ -250,11 +251,26 @@ def gather_kv(k_pool: torch.Tensor, v_pool: torch.Tensor, block_table: torch.Ten
     return kd, vd
 
 
-@functools.lru_cache(maxsize=256)   # of the shape alone
 def decode_workspace_bytes(num_seqs: int, hq: int, hkv: int, d: int, block_size: int,
                            max_seq_len: int, num_splits: int = 0) -> int:
     return lib().llkv_paged_decode_workspace_size(num_seqs, hq, hkv, d, block_size, max_seq_len,
                                                   num_splits)
+
+
+# Sizes remembered by shape, for plain integers alone: tensors and arrays, which the C call takes
+# as well, may change in place.
+@functools.lru_cache(maxsize=256)
+def _decode_size(*shape: int) -> int:
+    return lib().llkv_paged_decode_workspace_size(*shape)
+
+
+def _decode_workspace_bytes(num_seqs: int, hq: int, hkv: int, d: int, block_size: int, max_seq_len,
+                            num_splits) -> int:
+    if type(max_seq_len) is not int or type(num_splits) is not int:
+        return decode_workspace_bytes(num_seqs, hq, hkv, d, block_size, max_seq_len, num_splits)
+    if max_seq_len > 0 and block_size > 0:   # the size depends on the number of pages
+        max_seq_len -= (max_seq_len - 1) % block_size
+    return _decode_size(num_seqs, hq, hkv, d, block_size, max_seq_len, num_splits)
 
 
 DECODE_SCHEDULES = ("one_split", "unit", "splits", "balanced", "generic")
@@ -301,7 +317,7 @@ def paged_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
         scale = 1.0 / math.sqrt(d)
     if out is None:
         out = torch.empty_like(q)
-    ws = decode_workspace_bytes(b, hq, hkv, d, bs, max_seq_len, num_splits)
+    ws = _decode_workspace_bytes(b, hq, hkv, d, bs, max_seq_len, num_splits)
     if ws and (workspace is None or workspace.numel() * workspace.element_size() < ws):
         workspace = _workspace(ws, q.device)
     check(lib().llkv_paged_decode(_ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), _ptr(block_table),
@@ -330,7 +346,7 @@ def paged_decode_append(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tenso
         scale = 1.0 / math.sqrt(d)
     if out is None:
         out = torch.empty_like(q)
-    ws = decode_workspace_bytes(b, hq, hkv, d, bs, max_seq_len, num_splits)
+    ws = _decode_workspace_bytes(b, hq, hkv, d, bs, max_seq_len, num_splits)
     if ws and (workspace is None or workspace.numel() * workspace.element_size() < ws):
         workspace = _workspace(ws, q.device)
     check(lib().llkv_paged_decode_append(_ptr(out), _ptr(q), _ptr(k_new), _ptr(v_new), _ptr(k_pool),
@@ -352,9 +368,16 @@ def paged_attention(q: torch.Tensor, block_table: torch.Tensor, max_blocks_per_s
     return paged_decode(q, allocator.k_storage, allocator.v_storage, bt, seq_lens, max_seq_len)
 
 
-@functools.lru_cache(maxsize=256)   # of the shape alone
-def _prefill_workspace_bytes(*shape: int) -> int:
+@functools.lru_cache(maxsize=256)
+def _prefill_size(*shape: int) -> int:
     return lib().llkv_paged_prefill_workspace_size(*shape)
+
+
+def _prefill_workspace_bytes(num_seqs: int, total_q: int, max_q_len, max_seq_len, hq: int, d: int, block_size: int,
+                             dtype: int) -> int:
+    plain = type(max_q_len) is int and type(max_seq_len) is int
+    size = _prefill_size if plain else lib().llkv_paged_prefill_workspace_size
+    return size(num_seqs, total_q, max_q_len, max_seq_len, hq, d, block_size, dtype)
 
 
 def paged_prefill(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,

@@ -88,6 +88,32 @@ def test_decode_workspace_size():
     assert ws(64, 14, 2, 64, 16, 32768, 0) >= ws(64, 14, 2, 64, 16, 2048, 0)
 
 
+def test_python_sizes_follow_their_arguments():
+    """The sizes the Python operators ask for are those of the C call, also where a bound is a
+    tensor or an array that changes in place, and for every length of a page."""
+    import numpy as np
+    import torch
+
+    from lightllm_amd import kv_cache as kc
+
+    decode, prefill = L.lib().llkv_paged_decode_workspace_size, L.lib().llkv_paged_prefill_workspace_size
+    for make in (lambda: torch.tensor(64), lambda: np.array(64)):
+        bound = make()
+        for n in (64, 4096, 700):
+            bound[...] = n
+            assert kc.decode_workspace_bytes(64, 14, 2, 64, 16, bound) == decode(64, 14, 2, 64, 16, n, 0)
+        for n in (64, 4096, 700):
+            bound[...] = n
+            assert kc._decode_workspace_bytes(64, 14, 2, 64, 16, bound, 0) == decode(64, 14, 2, 64, 16, n, 0)
+            assert kc._prefill_workspace_bytes(2, 600, 300, bound, 14, 64, 16, 0) == prefill(2, 600, 300, n, 14, 64, 16, 0)
+    with pytest.raises(ctypes.ArgumentError):
+        kc.decode_workspace_bytes(64, 14, 2, 64, 16, 4096.0)
+    for bs in (1, 13, 16):
+        for n in [-5, 0, *range(1, 70), 1023, 1024, 1025, 32767, 32768]:
+            for splits in (0, 1, 7, 100):
+                assert kc._decode_workspace_bytes(9, 14, 2, 64, bs, n, splits) == decode(9, 14, 2, 64, bs, n, splits)
+
+
 def test_decode_rejects_small_workspace():
     lib = L.lib()
     need = lib.llkv_paged_decode_workspace_size(4, 14, 2, 64, 16, 4096, 8)
