@@ -58,9 +58,9 @@ struct MfmaPrefillArgs {
     float scale_log2;
     int qblocks;      // query blocks per sequence
     // Cut key ranges (pick_item): partial slots (0: nothing is cut), launched
-    // items beyond the units, tiles per chunk as a share of the sum of tiles.
-    int max_parts, extra_items;
-    float chunk_share;
+    // items beyond the units.
+    int max_parts, extra_items, cut_margin;
+    int groups;       // (item, kv head) pairs
     int2* table;      // per unit: first partial slot, chunks; from the main kernel to the merge
     float* part_o;    // [max_parts][Hq][BQ][D]
     float* part_lse;  // [max_parts][Hq][BQ]

@@ -112,23 +112,29 @@ __device__ inline UnitInfo unit_info(const MfmaPrefillArgs& a, int u) {
 // (descending, ties by index).  Every work-group derives the same items from the
 // same lengths; item y is the y-th chunk in that order.
 //
-// limit: no unit is cut when the longest has at most a compute unit's share of
-// the launch (sum of tiles x Hq / CUs): such loads run best unsplit (no
-// partials, no merge).  Otherwise the longest is cut into the fewest
-// equal chunks of at most kShare / 8 of a resident slot's share (at least
-// kMinChunkTiles), and the others to the same size.  The launched items and the
-// partial slots bound it too: a cut unit of t tiles has
-// ceil(t / limit) <= t / limit + 1 chunks, at most 2 t / limit, so
-// sum / limit <= extra items and 2 sum / limit <= slots suffice.
+// limit: no unit is cut unless the longest has cut_margin tiles more than a
+// compute unit's share of the launch (sum of tiles x Hq / CUs): partials and merge
+// cost that much (cut_margin(); cutting from the share on took 12/2/128 fp16 chunks of
+// 2, 1062, 23, 309, 808, 4 and 1496 rows from 42.7 to 52.9 us).
+// Otherwise the longest is cut into the fewest equal chunks of at most that share or
+// kMinChunkTiles, the greater, and the others to the same size.  With one
+// work-group per CU a second round waits for the first: there the limit is the
+// first up to 7/4 of the share at which the items run in one round (761 fp32 rows
+// on 1031, 16/8/256: 17 items per head 340 us, 16 items 277), or else 7/4 of it
+// (16/8/256 fp16 chunks of 1 .. 1121 rows 102 us cut at the share, 76 uncut).
+// The launched items and the partial slots bound the limit too: a cut unit of t
+// tiles has ceil(t / limit) < t / limit + 1 chunks, at most 2 t / limit, so
+// sum / limit <= extra items suffices, and for the slots either of
+// 2 sum / limit <= slots and sum / limit <= slots - units.  (The first alone cut
+// one unit of 54 tiles for 32/32/96 heads into four chunks of 14 where seven of 8
+// run in 24 us instead of 29.)
 //
 // pick_item leaves in LDS each unit's lengths, so that the chosen unit costs no
 // second global round trip; every thread of the work-group calls it (it contains
 // barriers).
 constexpr int kRankUnits = 1024;
 constexpr int kMinChunkTiles = 8;
-// 14/2/64 eight 512-row fp16 chunks on prefixes up to 4096: 62.6 us at 10 / 8,
-// 62.3 at 12, 58.6 at 14 and 16; the fp32 form 159 .. 160 at all four.
-constexpr int kShare = 14;
+constexpr int kFitUnits = 256;   // units up to which a limit that fits one round is looked for (0.4 us per 64)
 constexpr int kKeyTiles = (1 << 19) - 1;   // the ranking's key: 19 bits of tiles, 12 of chunks
 
 struct Item {
@@ -176,22 +182,39 @@ __device__ inline bool pick_item(const MfmaPrefillArgs& a, int y, int* lds, Item
     if (threadIdx.x == 0) s_item.unit = -1;
     __syncthreads();
     if (cut) {
-        int sum = 0, longest = 0;
+        int sum = 0, longest = 0, units = 0;
         for (int v = threadIdx.x & 63; v < U; v += 64) {   // every wave for itself
             const int t = max(tiles[v], 0);
             sum += t;
             longest = max(longest, t);
+            units += tiles[v] >= 0 ? 1 : 0;
         }
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
             sum += __shfl_xor(sum, off, 64);
             longest = max(longest, __shfl_xor(longest, off, 64));
+            units += __shfl_xor(units, off, 64);
         }
-        if ((int64_t)longest * a.n_cus > (int64_t)sum * a.Hq) {   // uniform
-            const int most = max(kMinChunkTiles, (int)ceilf((float)sum * a.chunk_share));
-            const int k = (longest + most - 1) / most;
-            const int limit = max((longest + k - 1) / k, max((2 * sum + a.max_parts - 1) / a.max_parts,
-                                                             (sum + a.extra_items - 1) / a.extra_items));
+        const int share = (int)(((int64_t)sum * a.Hq + a.n_cus - 1) / a.n_cus);
+        if ((int64_t)(longest - a.cut_margin) * a.n_cus > (int64_t)sum * a.Hq) {   // uniform
+            const bool one = a.resident < 2 * a.n_cus;
+            const int per = one ? (7 * share + 3) / 4 : share;
+            const int most = (longest + kMinChunkTiles - 1) / kMinChunkTiles;   // chunks of the longest
+            const int k = min((longest + per - 1) / per, most);
+            int limit = (longest + k - 1) / k;
+            if (one && units * a.Hq <= a.resident && U <= kFitUnits) {   // a lane per limit
+                const int l = max(share, (longest + most - 1) / most) + (threadIdx.x & 63);
+                const float inv = 1.0f / l;
+                int n = 0;
+                for (int v = 0; v < U; ++v)
+                    n += tiles[v] < 0 ? 0 : max(1, (int)((float)(tiles[v] + l - 1) * inv));
+                const uint64_t fits = __builtin_amdgcn_ballot_w64(n * a.Hq <= a.resident && l <= per);
+                if (fits != 0) limit = l - (int)(threadIdx.x & 63) + __builtin_ctzll(fits);
+            }
+            int by_slots = (2 * sum + a.max_parts - 1) / a.max_parts;
+            const int spare = a.max_parts - units;
+            if (spare > 0) by_slots = min(by_slots, (sum + spare - 1) / spare);
+            limit = max(limit, max(by_slots, (sum + a.extra_items - 1) / a.extra_items));
             for (int u = threadIdx.x; u < U; u += blockDim.x) {
                 const int t = tiles[u];
                 if (t > limit) {
@@ -275,14 +298,16 @@ __device__ inline bool take_work(const MfmaPrefillArgs& a, int* lds, Work& wk) {
     // Work-groups b, b + CUs, b + 2 CUs of the first resident set share a CU.
     // When a CU holds two or more, the second set takes its items in reverse,
     // so that the CU holding the longest item of the first set gets the
-    // shortest of the second.
+    // shortest of the second, or none: a grid of more than one set has two whole
+    // ones.  (With the reverse of a part of the second set the longest items got
+    // the others beside them, and the CUs of the shortest none: 28/4/128 fp16
+    // chunks of 1009, 11, 1 and 2 rows 30.4 -> 32.1 us.)
     int bid = blockIdx.x;
-    if (a.resident >= 2 * a.n_cus && bid >= a.n_cus && bid < 2 * a.n_cus) {
-        const int hi = min(2 * a.n_cus, (int)gridDim.x);
-        bid = a.n_cus + (hi - 1 - bid);
-    }
+    if (a.resident >= 2 * a.n_cus && bid >= a.n_cus && bid < 2 * a.n_cus)
+        bid = a.n_cus + (2 * a.n_cus - 1 - bid);
     const int xcd = bid % kXcds, r = bid / kXcds;
     const int j = (r / G) * kXcds + xcd;
+    if (j >= a.groups) return false;
     wk.kvh = j % a.Hkv;
     wk.hq = wk.kvh * G + r % G;
     Item it;
@@ -1829,14 +1854,16 @@ bool prefill_mfma_handles(int head_dim, int block_size, int dtype) {
 // prefixes up to 3000: 81 us, cut 86 .. 97).  Units are counted from the rows
 // (at most total_q / BQ + N hold any), not as N x the longest sequence's blocks:
 // 28/4/128 bf16 chunks of 64, 31, 700 and 5 rows 89 -> 38 us by that count.
-// Kernels of one work-group per CU (fp32 at head_dim 96 / 128, head_dim 256) cut
-// up to twice their slots: no second work-group runs beside a long one there
-// (32/8/128 fp32 chunks of 512, 300, 77 on 1000, 0, 2000: 288 heads' units, 169 ->
-// 120 us).
+// Kernels of one work-group per CU (fp32 at head_dim 96 / 128, head_dim 256) may cut
+// up to twice their slots: no second work-group runs beside a long one there.
+// A bound of the lengths that no unit can pass the rule of pick_item with (chunks
+// of max_q_len rows on no prefixes) saves the merge kernel's launch, 2 .. 3 us
+// (32/8/128 fp16 chunks of 1139, 226, 18, 2 and 10 rows 35.9 -> 32.9).
 // The workspace is sized for kSizingSlots resident slots (256 CUs x 4
 // work-groups, above what these kernels reach), so that it does not depend on
 // the device.
 constexpr int kSizingSlots = 1024;
+constexpr int kSizingItems = 512;   // items per head that cuts may add, above a device's CUs
 
 typedef void (*PrefillFn)(MfmaPrefillArgs);
 
@@ -1906,12 +1933,29 @@ ChunkPlan chunk_plan(int N, int Hq, int total_q, int max_q_len, int max_seq_len)
     c.extra = c.parts = 0;
     if (all <= kRankUnits && max_tiles >= 2 * kMinChunkTiles &&
         (int64_t)c.units * Hq < kSizingSlots) {
-        // sum / limit at the share, and a quarter more for the equal chunks
-        const int64_t share = (kSizingSlots * 10 + Hq * kShare - 1) / (Hq * kShare);
-        c.extra = (int)std::max<int64_t>(1, share);
-        c.parts = (int)std::max<int64_t>(2, std::min<int64_t>(2 * share, (int64_t)c.units * (max_tiles / kMinChunkTiles + 1)));
+        const int64_t share = (kSizingItems + Hq - 1) / Hq;   // at least sum / limit (pick_item)
+        c.extra = (int)share;
+        c.parts = (int)std::max<int64_t>(2, std::min<int64_t>(2 * share, (int64_t)c.units * ((max_tiles - 1) / kMinChunkTiles + 2)));
     }
     return c;
+}
+
+// Key tiles of total_q rows in chunks of max_q_len on no prefixes.
+int64_t causal_tiles(int total_q, int max_q_len) {
+    const int64_t rows = (max_q_len > 0 && max_q_len < total_q) ? max_q_len : total_q;
+    auto tiles = [](int64_t n) {   // 2, 4, .. of the whole query blocks, and the last
+        const int64_t m = n / BQ;
+        return m * (m + 1) + (n % BQ != 0 ? (n + BN - 1) / BN : 0);
+    };
+    return total_q / rows * tiles(rows) + tiles(total_q % rows);
+}
+
+// Tiles that cutting has to save (pick_item): a merge and the partials, whose bytes
+// grow with head_dim, over a tile's time.  Of 475 random batches of every type and
+// head_dim the slower of cut and uncut is taken by 1.1x at most so; by one margin of
+// 4 tiles, 1.2x (16 bits at head_dim 128), of 16, 1.9x (fp32 at 256).
+int cut_margin(int dtype, int head_dim) {
+    return dtype == LLKV_DTYPE_F32 ? head_dim / 32 : 6 + head_dim / 64;
 }
 
 size_t part_bytes(int Hq, int head_dim) { return (size_t)Hq * BQ * (1 + head_dim) * sizeof(float); }
@@ -1942,12 +1986,14 @@ int launch_prefill_mfma(MfmaPrefillArgs a, int head_dim, int block_size, int dty
     a.extra_items = 0;
     a.table = nullptr;
     a.part_lse = a.part_o = nullptr;
+    a.cut_margin = cut_margin(dtype, head_dim);
     const int cut_below = a.resident < 2 * a.n_cus ? 2 * a.resident : a.resident;
-    if (need > 0 && (int64_t)c.units * a.Hq < cut_below && workspace != nullptr &&
+    const int64_t max_tiles = (std::max(max_seq_len, 1) + BN - 1) / BN;
+    const bool uneven = !a.causal || (max_tiles - a.cut_margin) * a.n_cus > causal_tiles(total_q, max_q_len) * a.Hq;
+    if (need > 0 && uneven && (int64_t)c.units * a.Hq < cut_below && workspace != nullptr &&
         workspace_bytes >= need) {
         a.max_parts = c.parts;
         a.extra_items = c.extra;
-        a.chunk_share = (float)kShare / 8.0f * a.Hq / std::min(a.resident, kSizingSlots);
         char* base = reinterpret_cast<char*>(workspace) + kPlanHeaderBytes;
         const size_t rows = (size_t)c.parts * a.Hq * BQ;
         a.part_lse = reinterpret_cast<float*>(base);
@@ -1958,7 +2004,10 @@ int launch_prefill_mfma(MfmaPrefillArgs a, int head_dim, int block_size, int dty
     const int64_t all = (int64_t)a.N * a.qblocks;
     const int64_t groups = (all > kRankUnits ? all : c.units + a.extra_items) * a.Hkv;
     const int G = a.Hq / a.Hkv;
-    dim3 grid((unsigned)(((groups + kXcds - 1) / kXcds) * kXcds * G));
+    a.groups = (int)groups;
+    int64_t wgs = ((groups + kXcds - 1) / kXcds) * kXcds * G;
+    if (a.resident >= 2 * a.n_cus && wgs > a.n_cus) wgs = std::max<int64_t>(wgs, 2 * a.n_cus);   // take_work
+    dim3 grid((unsigned)wgs);
     prefill_kernel(dtype, head_dim, a.contig != 0)<<<grid, 256, 0, st>>>(a);
     if (a.max_parts > 0)
         merge_kernel(dtype, head_dim)<<<dim3(a.Hq, a.N * a.qblocks), 256, 0, st>>>(a);

@@ -270,6 +270,41 @@ def test_prefill_work_items(name, dtype):
         assert torch.all((got - ref).abs() <= bar), (i, float(((got - ref).abs() / bar).max()))
 
 
+# How a launch cuts key ranges, from the chunk counts that it leaves for the merge kernel in the
+# workspace's last slot (one query block per chunk here, so unit n is sequence n): one long unit fills
+# the GPU in chunks of at least 8 tiles; batches whose longest unit is near a compute unit's share are
+# not cut; kernels of one work-group per CU take as many chunks as run at once.
+CUTS = [
+    ("one_unit", torch.float16, 32, 32, 96, [66], [3381], [7]),              # 54 tiles: seven of eight
+    ("one_unit_d256", torch.float16, 16, 8, 256, [63], [4125], [9]),         # 66 tiles: nine
+    ("near_share", torch.float16, 32, 8, 128, [128] * 7, [1100] * 6 + [1500], None),
+    ("long_beside_short", torch.float16, 32, 8, 128, [3, 40], [200, 2000], [1, 4]),   # 32 tiles
+    ("one_round", torch.float32, 16, 8, 256, [128] * 6, [1031, 1159, 1287, 1415, 1543, 1671], [2, 2, 3, 3, 3, 3]),
+]
+
+
+@pytest.mark.parametrize("name,dtype,hq,hkv,d,chunks,prefixes,want", CUTS, ids=[c[0] for c in CUTS])
+def test_prefill_cut_counts(name, dtype, hq, hkv, d, chunks, prefixes, want):
+    totals = [p + c for p, c in zip(prefixes, chunks)]
+    n, width = len(chunks), (max(totals) + 15) // 16
+    pool = torch.zeros(width, 16, hkv, d, dtype=dtype, device=DEV)
+    table = torch.arange(width, dtype=torch.int32, device=DEV).repeat(n, 1)
+    q = torch.zeros(sum(chunks), hq, d, dtype=dtype, device=DEV)
+    cu = torch.tensor([0] + torch.tensor(chunks).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    size = kc.lib().llkv_paged_prefill_workspace_size(n, sum(chunks), max(chunks), max(totals), hq, d, 16,
+                                                      kc.dtype_code(dtype))
+    ws = torch.full((size,), 255, dtype=torch.uint8, device=DEV)
+    out = kc.paged_prefill(q, pool, pool, table, cu, torch.tensor(totals, dtype=torch.int32, device=DEV),
+                           max(chunks), max(totals), workspace=ws)
+    assert torch.all(out == 0)
+    slot = hq * 128 * (1 + d) * 4
+    counts = ws[size - slot:size - slot + 8 * n].view(torch.int32)[1::2].tolist()
+    if want is None:
+        assert all(c in (-1, 1) for c in counts), counts   # -1: the host did not let it cut
+    else:
+        assert counts == want
+
+
 # Balanced decode: a unit cut into exactly the merge's four entries per trip, fewer, more, and many
 # (one sequence of nearly all pages), beside short sequences inside one share.
 @pytest.mark.parametrize("d,hq,hkv", [(64, 14, 2), (128, 32, 8), (256, 16, 8)])
