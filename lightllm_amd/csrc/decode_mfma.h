@@ -326,8 +326,12 @@ struct MfmaDecode {
                 }
             }
             // The fused variant's pointer selects make the scheduler sink the V
-            // loads next to their MFMAs; keep all of the page's loads first.
-            if constexpr (A) __builtin_amdgcn_sched_barrier(0);
+            // loads next to their MFMAs, and so it does at head_dim 256 in 16 bits
+            // for a third wave per SIMD; keep all of the page's loads first.  (200 x
+            // 258 .. 516 tokens of 16/8/256 bf16 113 us, sunk 123.  fp16 stays sunk:
+            // the same gain there, but 81 x 46 .. 92 tokens 12.6 -> 14.6 us.)
+            constexpr bool kBf16 = Elem<T>::kDtype == LLKV_DTYPE_BF16;
+            if constexpr (A || (kHalfPV && kBf16)) __builtin_amdgcn_sched_barrier(0);
 
             const mf32x4 sacc = Ops::scores(kr, qop, a.scale_log2);
             const int t0 = pg * kPage + 4 * g;
