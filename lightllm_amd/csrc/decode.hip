@@ -143,10 +143,15 @@ __global__ __launch_bounds__(64) void decode_generic_kernel(DecodeArgs a) {
 // balanced schedule, whose units are mostly cut in two or three (16 issues up to
 // 64 masked loads a lane for them): 61 x 100 .. 2100 tokens of 16/8/256 bf16 120
 // -> 106 us a call, 256 lognormal contexts of 32/8/128 fp16 388 -> 385; 2 and 8
-// measured the same as 4.
+// measured the same as 4.  Up to head_dim 64 its units of more than kFewEntries
+// take 16 as well: 131072 tokens of 14/2/64 fp16 beside 299 x 50 .. 300, over a hundred
+// entries, 69 us by 16, 91 by 4.  (Not beyond: with both forms the kernel's registers
+// cost more, 32768 tokens beside 63 short ones of 16/8/256 84 us by 4, 121.)
 // The reference's paged_attention_reduce_kernel
 // (src/kv_cache/paged_attention.cu:477-532) computes the same sum in
 // unnormalised form: out = sum_j 2^(lse_j - M) o_j / sum_j 2^(lse_j - M).
+constexpr int kFewEntries = 8;
+
 template <typename T, int MD, int kMergeBatch, class Live>
 __device__ inline void merge_partials(const float* po, int64_t po_step, const float* pl,
                                       int64_t pl_step, int count, int D, Live live, T* out) {
@@ -236,10 +241,17 @@ __global__ __launch_bounds__(1024) void decode_merge_balanced_kernel(DecodeArgs 
     const float* po = a.part_o + (seg0 * G + h) * D;
     const float* pl = a.part_lse + seg0 * G + h;
     const int cnt = (int)(wl - wf + 1);
-    if (T_ >= a.nwg)   // every work-group holds pages: all entries live
-        merge_partials<T, MD, 4>(po, (int64_t)G * D, pl, G, cnt, D, AllLive(), out);
-    else
-        merge_partials<T, MD, 4>(po, (int64_t)G * D, pl, G, cnt, D, LiveWG{wf, T_, a.nwg}, out);
+    auto merge = [&](auto live) {
+        if constexpr (MD == 1) {
+            if (cnt > kFewEntries) {   // the same for every lane
+                merge_partials<T, MD, 16>(po, (int64_t)G * D, pl, G, cnt, D, live, out);
+                return;
+            }
+        }
+        merge_partials<T, MD, 4>(po, (int64_t)G * D, pl, G, cnt, D, live, out);
+    };
+    if (T_ >= a.nwg) merge(AllLive());   // every work-group holds pages
+    else merge(LiveWG{wf, T_, a.nwg});
 }
 
 // ---------------------------------------------------------------------------
