@@ -33,6 +33,7 @@ struct DecodeArgs {
     // and reads that token from here instead of the pool.
     const void* knew;
     const void* vnew;
+    int64_t stream_units;   // page-units from which K and V are streamed (decode_sched.h)
 };
 
 // Split geometry of one sequence; identical in the split and merge kernels.

@@ -257,18 +257,23 @@ __global__ __launch_bounds__(1024) void decode_merge_balanced_kernel(DecodeArgs 
 // ---------------------------------------------------------------------------
 // Host dispatch
 // ---------------------------------------------------------------------------
-// K/V bytes (by the shape bounds) from which a batch is read with streaming
-// loads: three quarters of the 256 MB last-level cache.  Such a batch finds
-// nothing of itself there on the next call, and loads that do not allocate run
-// faster (256 lognormal contexts of 32/8/128 fp16 390 -> 365 us, 16 x 32768 of
-// 14/2/64 fp16 56 -> 53, 61 x 100 .. 2100 of 16/8/256 bf16 106 -> 99); smaller
-// batches may stay cached (64 x 129 .. 2049 of 14/2/64 fp32, 134 MB: 23.6 us, by
-// streaming loads 24.6).
+// K/V bytes from which a batch is read with streaming loads: three quarters of the
+// 256 MB last-level cache.  Between one layer's call and its next the other layers'
+// pools pass through that cache, so such a batch finds little of itself there, and
+// loads that do not allocate run faster (two pools in turn: 32 x 1048 .. 2096 tokens
+// of 32/8/128 bf16, 211 MB, 49.5 -> 47.8 us; 256 x 1048 .. 2096 of 14/2/64 fp16 55.8 ->
+// 48.4; 32 x 524 .. 1048 of 16/8/256 bf16 51.1 -> 43.4).  One pool again and again stays
+// partly cached up to about 340 MB: 44.3 -> 48.6, 50.1 -> 48.3 and 47.0 -> 44.3.
+// The host takes the kernels that may stream by the shape bounds, and they decide by
+// the actual lengths and shared pages (decode_sched.h).
 // Instantiated where it measured faster: the balanced schedule at head_dim 64
 // (93 -> 86 us bf16, 99 -> 90 fp32), 256 (also 144 -> 128 fp32), 128 in 16 bits
-// and 96 in fp32 (183 -> 171), and the 16-wave splits at head_dim 64 in 16 bits.
-// Slower and left plain: fp32 at head_dim 128 (172 -> 194), 16 bits at 96 (252 ->
-// 256), the 16-wave splits at 128 (116 -> 127) and in fp32 (70.5 -> 74.8).
+// (not the fused append) and 96 in fp32 (183 -> 171), and the 16-wave splits at
+// head_dim 64 in 16 bits.  Slower and left plain, on one or two shapes each: fp32 at
+// head_dim 128 (172 -> 194), 16 bits at 96 (252 -> 256), the 16-wave splits at 128 (116
+// -> 127) and in fp32 (70.5 -> 74.8), and the fused append at head_dim 128, where the
+// two forms of the page loop spill (256 lognormal contexts of 32/8/128 fp16 393 -> 385,
+// but 71 x 127 .. 2044 tokens 69 -> 73).
 constexpr int64_t kStreamBytes = 192ll << 20;
 
 // The tuned kernels of a pool type, plain or fused-append (decode_tuned_*.hip).
@@ -595,6 +600,7 @@ int paged_decode_impl(const char* fn, void* out, const void* q, const void* k_ne
     a.plan = nullptr;
     a.knew = k_new;
     a.vnew = v_new;
+    a.stream_units = kStreamBytes / ((int64_t)kPage * head_dim * 2 * (int64_t)es);
     char* ws = reinterpret_cast<char*>(workspace);
     hipStream_t st = (hipStream_t)stream;
 

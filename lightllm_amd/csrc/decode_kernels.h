@@ -26,8 +26,8 @@ struct Kernels {
 Kernels tuned_kernels_f32(int D, int G, bool append);
 Kernels tuned_kernels_f16(int D, int G, bool append);
 Kernels tuned_kernels_bf16(int D, int G, bool append);
-// The same kernels with streaming (nontemporal) loads of K and V, those that
-// measured faster so; the others null.
+// Kernels that may stream K and V (nontemporal loads), where that measured faster;
+// the others null.
 Kernels tuned_kernels_f32_stream(int D, int G, bool append);
 Kernels tuned_kernels_f16_stream(int D, int G, bool append);
 Kernels tuned_kernels_bf16_stream(int D, int G, bool append);

@@ -158,14 +158,14 @@ template <int D> struct ScoreOps<bf16_t, D> : ScoreOps16<bf16_t, D> {};
 // loop has no trace of it.
 // WV: waves per work-group (kDecodeWaves; kUnitWaves for the one-work-group-
 // per-unit schedule of small batches).
-// NT: K and V by nontemporal loads, for batches beyond the last-level cache
-// (kStreamBytes, decode.hip).
-template <typename TT, int D, int G, bool A = false, int WV = kDecodeWaves, bool NT = false>
+// ST: the kernel chooses between plain and streaming (nontemporal) loads of K and
+// V (decode_sched.h), for batches that may be beyond the last-level cache.
+template <typename TT, int D, int G, bool A = false, int WV = kDecodeWaves, bool ST = false>
 struct MfmaDecode {
     static_assert(G >= 1 && G <= 16, "up to 16 query heads per KV head");
     static_assert(D % 32 == 0, "head_dim multiple of 32");
     using T = TT;
-    static constexpr bool kStream = NT;
+    static constexpr bool kStream = ST;
     using Ops = ScoreOps<T, D>;
     static constexpr int W = WV;              // waves per work-group
     static constexpr int kThreads = 64 * W;
@@ -202,9 +202,15 @@ struct MfmaDecode {
         float ml[kSegMax][W][G][2];   // (max, sum); sum 0: the wave had no page
     };
 
+    // NT: nontemporal loads of K and V
+    template <bool NT>
     __device__ static void round(const DecodeArgs& a, Smem& sm, const SegDesc* segs, int nseg,
                                  int64_t po_stride, int64_t pl_stride) {
-        const int tid = threadIdx.x, lane = tid & 63;
+        const int tid = threadIdx.x;
+        int lane = tid & 63;
+        // (opaque: without it the two forms of the loop share lane offsets, 256 x 1025 ..
+        // 1124 tokens of 14/2/64 fp16 on one prefix 40 -> 44 us)
+        if constexpr (ST && D == 64 && !A) asm volatile("" : "+v"(lane));
         const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index, known uniform
         const int g = lane >> 4, c = lane & 15;
         const int np_total = segs[nseg - 1].cum + segs[nseg - 1].npages;

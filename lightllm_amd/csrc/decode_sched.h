@@ -11,6 +11,25 @@
 namespace llkv {
 namespace {
 
+// Streaming (nontemporal) loads, in the kernels that may use them (Body::kStream;
+// kStreamBytes in decode.hip): for batches that read more than stream_units
+// page-units by their actual lengths, and segments whose middle page is no other
+// sequence's too.  A page that several sequences read (a cached prefix) is read
+// again from the caches, where streaming loads leave nothing: 256 sequences of
+// 32/8/128 fp16 on one prefix of 2048 tokens 265 us, 332 streamed.  A prefix lies at
+// the same place of each table, so one entry per sequence tells.  The choice costs 1
+// to 2 us: 16 x 32768 tokens of 14/2/64 fp16 51.3 -> 52.6, 55.8 without streaming loads.
+// shares_page: whether this lane's part (of `lanes`) of the other sequences has page
+// pg of sequence b.
+template <class Pages>
+__device__ inline bool shares_page(const DecodeArgs& a, int b, int pg, int lane, int lanes, Pages pages) {
+    const int id = a.bt[(int64_t)b * a.max_blocks + pg];
+    bool same = false;
+    for (int j = lane; j < a.B; j += lanes)
+        same |= (a.bt[(int64_t)j * a.max_blocks + pg] == id) & (pages(j) > pg) & (j != b);
+    return same;
+}
+
 // Fixed split schedule: grid (S_max, Hkv, B), Body::W waves per work-group,
 // one segment each.
 template <class Body>
@@ -46,9 +65,33 @@ void decode_split_kernel(DecodeArgs a) {
         d.po_off = (bh0 * a.S_max + split) * a.D;
         d.pl_off = bh0 * a.S_max + split;
     }
+    bool stream = false;   // the same in every wave
+    if constexpr (Body::kStream) {
+        // (as if every sequence were as long, so that small batches under a large
+        // bound load nothing here; then the actual lengths)
+        if ((int64_t)geo.npages * a.B * a.Hkv > a.stream_units) {
+            const int lane = threadIdx.x & 63;
+            const int pg = split * geo.pps, n = min(geo.pps, geo.npages - pg);
+            const int warm = a.bt[(int64_t)b * a.max_blocks + pg + min((int)threadIdx.x, n - 1)];   // for round()
+            auto pages = [&](int j) { return (clamp_len(a, j) + kPage - 1) / kPage; };
+            int64_t units = 0;
+            for (int j = lane; j < a.B; j += 64) units += pages(j);
+            const bool same = shares_page(a, b, pg + n / 2, lane, 64, pages);
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) units += __shfl_xor(units, off, 64);
+            stream = units * a.Hkv > a.stream_units && __builtin_amdgcn_ballot_w64(same) == 0;
+            asm volatile("" ::"v"(warm));
+        }
+    }
     __syncthreads();
     store_new_row<T, Body::HD>(a, segs[0]);
-    Body::round(a, sm, segs, 1, (int64_t)a.S_max * a.D, a.S_max);
+    if constexpr (Body::kStream) {
+        if (stream) {
+            Body::template round<true>(a, sm, segs, 1, (int64_t)a.S_max * a.D, a.S_max);
+            return;
+        }
+    }
+    Body::template round<false>(a, sm, segs, 1, (int64_t)a.S_max * a.D, a.S_max);
 }
 
 // Balanced schedule: grid (nwg), 4 waves per work-group.  Every work-group
@@ -67,7 +110,7 @@ void decode_balanced_kernel(DecodeArgs a) {
     __shared__ int sP[kBalanceMaxB + 1];
     __shared__ int sL[kBalanceMaxB];
     __shared__ SegDesc segs[Body::kSegMax];
-    __shared__ int s_n;
+    __shared__ int s_n, s_shared;
     __shared__ int64_t s_next;
     LLKV_TRACE_POINT(0);
     scan_pages(a, sP, sL);
@@ -84,17 +127,37 @@ void decode_balanced_kernel(DecodeArgs a) {
     }
     const int64_t r1 = share_begin(wg + 1, T_, a.nwg);
     int64_t p = share_begin(wg, T_, a.nwg);
+    int stream = -1;   // not decided
     while (p < r1) {
         if (tid == 0) {
             int n = 0;
             s_next = build_segments(a, sP, sL, p, r1, wg, Body::kSegMax, segs, &n);
             s_n = n;
+            s_shared = 0;
         }
         __syncthreads();
         const int n = s_n;
         p = s_next;
         for (int i = 0; i < n; ++i) store_new_row<T, D>(a, segs[i]);
-        Body::round(a, sm, segs, n, D, 1);   // ends with a barrier
+        if constexpr (Body::kStream) {
+            if (T_ > a.stream_units && stream < 0) {   // uniform; by the share's first segments
+                const SegDesc& d = segs[0];
+                const int warm = a.bt[(int64_t)d.b * a.max_blocks + d.pg_begin + min(tid, d.npages - 1)];   // for round()
+                bool same = false;
+                for (int i = 0; i < n; ++i)
+                    same |= shares_page(a, segs[i].b, segs[i].pg_begin + segs[i].npages / 2, tid, blockDim.x,
+                                        [&](int j) { return sP[j + 1] - sP[j]; });
+                asm volatile("" ::"v"(warm));
+                if (same) s_shared = 1;
+                __syncthreads();
+                stream = s_shared == 0;
+            }
+            if (stream > 0) {
+                Body::template round<true>(a, sm, segs, n, D, 1);   // ends with a barrier
+                continue;
+            }
+        }
+        Body::template round<false>(a, sm, segs, n, D, 1);   // ends with a barrier
     }
 }
 
@@ -109,56 +172,59 @@ Kernels kernels_of() {
 // head_dim 64 / 128 also get the unit schedule's kUnitWaves-wave kernel,
 // except fp32 at head_dim 128, whose body does not fit the 128 registers of
 // four waves per SIMD (~50 would spill).
-template <typename T, int D, int G, bool A, bool NT>
+template <typename T, int D, int G, bool A, bool ST>
 Kernels kernels_with_unit() {
-    Kernels k = kernels_of<MfmaDecode<T, D, G, A, kDecodeWaves, NT>>();
+    Kernels k = kernels_of<MfmaDecode<T, D, G, A, kDecodeWaves, ST>>();
     constexpr bool kF32 = Elem<T>::kDtype == LLKV_DTYPE_F32;
-    if constexpr (!(kF32 && D == 128) && (!NT || (D == 64 && !kF32)))
-        k.unit = decode_split_kernel<MfmaDecode<T, D, G, A, kUnitWaves, NT>>;
+    if constexpr (!(kF32 && D == 128) && (!ST || (D == 64 && !kF32)))
+        k.unit = decode_split_kernel<MfmaDecode<T, D, G, A, kUnitWaves, ST>>;
     return k;
 }
 
-template <typename T, int D, bool A, bool NT>
+template <typename T, int D, bool A, bool ST>
 Kernels tuned_g(int G) {
     switch (G) {
-        case 1: return kernels_with_unit<T, D, 1, A, NT>();
-        case 2: return kernels_with_unit<T, D, 2, A, NT>();
-        case 3: return kernels_with_unit<T, D, 3, A, NT>();
-        case 4: return kernels_with_unit<T, D, 4, A, NT>();
-        case 5: return kernels_with_unit<T, D, 5, A, NT>();
-        case 6: return kernels_with_unit<T, D, 6, A, NT>();
-        case 7: return kernels_with_unit<T, D, 7, A, NT>();
-        case 8: return kernels_with_unit<T, D, 8, A, NT>();
-        case 12: return kernels_with_unit<T, D, 12, A, NT>();
-        case 16: return kernels_with_unit<T, D, 16, A, NT>();
+        case 1: return kernels_with_unit<T, D, 1, A, ST>();
+        case 2: return kernels_with_unit<T, D, 2, A, ST>();
+        case 3: return kernels_with_unit<T, D, 3, A, ST>();
+        case 4: return kernels_with_unit<T, D, 4, A, ST>();
+        case 5: return kernels_with_unit<T, D, 5, A, ST>();
+        case 6: return kernels_with_unit<T, D, 6, A, ST>();
+        case 7: return kernels_with_unit<T, D, 7, A, ST>();
+        case 8: return kernels_with_unit<T, D, 8, A, ST>();
+        case 12: return kernels_with_unit<T, D, 12, A, ST>();
+        case 16: return kernels_with_unit<T, D, 16, A, ST>();
     }
     return Kernels();
 }
 
 // head_dim 96 (Phi-3 layouts) and 256 (Gemma-2 / Gemma-3 layouts): group
 // sizes 1, 2, 4, 8.
-template <typename T, int D, bool A, bool NT>
+template <typename T, int D, bool A, bool ST>
 Kernels tuned_g_few(int G) {
     switch (G) {
-        case 1: return kernels_of<MfmaDecode<T, D, 1, A, kDecodeWaves, NT>>();
-        case 2: return kernels_of<MfmaDecode<T, D, 2, A, kDecodeWaves, NT>>();
-        case 4: return kernels_of<MfmaDecode<T, D, 4, A, kDecodeWaves, NT>>();
-        case 8: return kernels_of<MfmaDecode<T, D, 8, A, kDecodeWaves, NT>>();
+        case 1: return kernels_of<MfmaDecode<T, D, 1, A, kDecodeWaves, ST>>();
+        case 2: return kernels_of<MfmaDecode<T, D, 2, A, kDecodeWaves, ST>>();
+        case 4: return kernels_of<MfmaDecode<T, D, 4, A, kDecodeWaves, ST>>();
+        case 8: return kernels_of<MfmaDecode<T, D, 8, A, kDecodeWaves, ST>>();
     }
     return Kernels();
 }
 
-// NT: the streaming kernels, where they measured faster (kStreamBytes in
+// ST: the kernels that may stream, where they measured faster (kStreamBytes in
 // decode.hip); the others stay null and the plain ones run.
-template <typename T, bool NT>
+template <typename T, bool ST>
 Kernels tuned(int D, int G, bool append) {
     constexpr bool kF32 = Elem<T>::kDtype == LLKV_DTYPE_F32;
-    if (D == 64) return append ? tuned_g<T, 64, true, NT>(G) : tuned_g<T, 64, false, NT>(G);
-    if constexpr (!NT || !kF32)
-        if (D == 128) return append ? tuned_g<T, 128, true, NT>(G) : tuned_g<T, 128, false, NT>(G);
-    if (D == 256) return append ? tuned_g_few<T, 256, true, NT>(G) : tuned_g_few<T, 256, false, NT>(G);
-    if constexpr (!NT || kF32)
-        if (D == 96) return append ? tuned_g_few<T, 96, true, NT>(G) : tuned_g_few<T, 96, false, NT>(G);
+    if (D == 64) return append ? tuned_g<T, 64, true, ST>(G) : tuned_g<T, 64, false, ST>(G);
+    if constexpr (!ST) {
+        if (D == 128) return append ? tuned_g<T, 128, true, false>(G) : tuned_g<T, 128, false, false>(G);
+    } else if constexpr (!kF32) {
+        if (D == 128 && !append) return tuned_g<T, 128, false, true>(G);
+    }
+    if (D == 256) return append ? tuned_g_few<T, 256, true, ST>(G) : tuned_g_few<T, 256, false, ST>(G);
+    if constexpr (!ST || kF32)
+        if (D == 96) return append ? tuned_g_few<T, 96, true, ST>(G) : tuned_g_few<T, 96, false, ST>(G);
     return Kernels();
 }
 
