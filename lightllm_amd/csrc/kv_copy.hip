@@ -104,6 +104,8 @@ __device__ inline void copy_unit(char* kd, char* vd, const char* ks, const char*
     }
 }
 
+constexpr int64_t kGatherStreamBytes = 288ll << 20;   // launch_copy
+
 template <bool NT, typename U, typename Map>
 __global__ __launch_bounds__(256) void copy_rows_kernel(
     Map map, char* __restrict__ k_dst, char* __restrict__ v_dst,
@@ -146,12 +148,14 @@ int launch_copy(const char* what, Map map, void* kd, void* vd, const void* ks,
     char* v_d = (char*)vd;
     const char* k_s = (const char*)ks;
     const char* v_s = (const char*)vs;
-    // Gathers that read and write more than three quarters of the 256 MB last-level
-    // cache stream past it: 70 k rows of 8 x 128 bf16 (572 MB) 132 -> 122 us, but
-    // 148 MB 36.3 -> 37.1.  The scatters' rows are read again by the attention that
-    // follows (a first prefill 38.6 -> 41.8 us with streaming copies).
+    // Gathers that read and write more than 9/8 of the 256 MB last-level cache stream
+    // past it (three sets of buffers in turn, 14/2/64 fp16: 300 MB 72.8 -> 71.0 us, 340 MB
+    // 84.7 -> 79.1, 1000 MB 229 -> 214, but 210 MB 49.1 -> 50.4 and 270 MB 61.8 -> 63.3; one
+    // set again and again, 209 MB of 32/8/128 fp32, 34.7 -> 52.2).  The scatters' rows are
+    // read again by the attention that follows (a first prefill 38.6 -> 41.8 us with
+    // streaming copies).
     if constexpr (std::is_same<Map, GatherMap>::value) {
-        if (unit == 16 && 4 * n_rows * row_bytes > (192ll << 20)) {
+        if (unit == 16 && 4 * n_rows * row_bytes > kGatherStreamBytes) {
             copy_rows_kernel<true, uint4><<<grid, block, 0, st>>>(map, k_d, v_d, k_s, v_s, n_rows, upr);
             return check_launch(what);
         }

@@ -442,9 +442,9 @@ def test_decode_shared_prefix_stays_cached():
 
 @pytest.mark.parametrize("extra", [0, 5])
 def test_gather_streaming_edge(extra):
-    """Gathers on both sides of the streaming rule (4 x rows x row bytes at 192 MB), bit for bit."""
+    """Gathers on both sides of the streaming rule (4 x rows x row bytes at 288 MB), bit for bit."""
     hkv, d = 8, 128
-    n = (192 << 20) // (4 * hkv * d * 2) + extra
+    n = (288 << 20) // (4 * hkv * d * 2) + extra
     g = torch.Generator(device=DEV).manual_seed(5)
     lens = [n // 3, n - n // 3 - 1, 1]
     need = [(x + 15) // 16 for x in lens]
