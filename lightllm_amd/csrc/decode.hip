@@ -268,12 +268,14 @@ __global__ __launch_bounds__(1024) void decode_merge_balanced_kernel(DecodeArgs 
 // the actual lengths and shared pages (decode_sched.h).
 // Instantiated where it measured faster: the balanced schedule at head_dim 64
 // (93 -> 86 us bf16, 99 -> 90 fp32), 256 (also 144 -> 128 fp32), 128 in 16 bits
-// (not the fused append) and 96 in fp32 (183 -> 171), and the 16-wave splits at
-// head_dim 64 in 16 bits.  Slower and left plain, on one or two shapes each: fp32 at
-// head_dim 128 (172 -> 194), 16 bits at 96 (252 -> 256), the 16-wave splits at 128 (116
-// -> 127) and in fp32 (70.5 -> 74.8), and the fused append at head_dim 128, where the
-// two forms of the page loop spill (256 lognormal contexts of 32/8/128 fp16 393 -> 385,
-// but 71 x 127 .. 2044 tokens 69 -> 73).
+// and 96 in fp32 (183 -> 171), and the 16-wave splits at head_dim 64 in 16 bits.
+// Slower and left plain, on one or two shapes each: fp32 at head_dim 128 (172 -> 194),
+// 16 bits at 96 (252 -> 256), the 16-wave splits at 128 (116 -> 127) and in fp32 (70.5
+// -> 74.8).
+// The fused append at head_dim 128 in 16 bits has no registers for two forms of its
+// page loop (20 spilled).  Beyond this bound its rows are appended by a kernel of
+// their own and the plain call's kernels decode: 256 lognormal contexts of 32/8/128
+// fp16 389 -> 358 us, 128 x 50 .. 200 tokens under a bound of 16384 33 -> 31.
 constexpr int64_t kStreamBytes = 192ll << 20;
 
 // The tuned kernels of a pool type, plain or fused-append (decode_tuned_*.hip).
@@ -495,9 +497,10 @@ extern "C" size_t llkv_paged_decode_workspace_size(int num_seqs, int num_q_heads
 namespace llkv {
 namespace {
 
-// Fused append on the generic path: the new K/V row of (sequence, kv head) =
-// (blockIdx.y, blockIdx.x) goes to position len - 1 before the decode kernel
-// runs (any head_dim and page size).
+// Fused append by a kernel of its own, for the generic decode and where the plain
+// kernels stream (kStreamBytes): the new K/V row of (sequence, kv head) =
+// (blockIdx.y, blockIdx.x) goes to position len - 1 before the decode kernel runs
+// (any head_dim and page size).
 template <typename T>
 __global__ __launch_bounds__(64) void append_new_rows_kernel(DecodeArgs a) {
     const int kvh = blockIdx.x, b = blockIdx.y;
@@ -513,6 +516,15 @@ __global__ __launch_bounds__(64) void append_new_rows_kernel(DecodeArgs a) {
         kp[dst + d] = reinterpret_cast<const T*>(a.knew)[src + d];
         vp[dst + d] = reinterpret_cast<const T*>(a.vnew)[src + d];
     }
+}
+
+// Launches it; the decode that follows takes the rows from the pools.
+void launch_append(int num_kv_heads, int num_seqs, int dtype, hipStream_t st, DecodeArgs& a) {
+    const dim3 grid(num_kv_heads, num_seqs);
+    if (dtype == LLKV_DTYPE_F32) append_new_rows_kernel<float><<<grid, 64, 0, st>>>(a);
+    else if (dtype == LLKV_DTYPE_F16) append_new_rows_kernel<_Float16><<<grid, 64, 0, st>>>(a);
+    else append_new_rows_kernel<bf16_t><<<grid, 64, 0, st>>>(a);
+    a.knew = a.vnew = nullptr;
 }
 
 // The schedule of a call: balanced, or fixed splits (num_splits updated to
@@ -575,11 +587,19 @@ int paged_decode_impl(const char* fn, void* out, const void* q, const void* k_ne
     const Kernels sched = (k_new != nullptr && ks.split != nullptr) ? pick_tuned(dtype, head_dim, G, false) : ks;
     decide_schedule(sched, num_seqs, num_kv_heads, block_size, max_seq_len, num_splits, balanced, wide);
 
+    bool append_first = false;   // a fused append in two kernels
     if (ks.split != nullptr &&
         (int64_t)num_seqs * max_seq_len * num_kv_heads * head_dim * 2 * (int64_t)es > kStreamBytes) {
         const Kernels st = pick_tuned(dtype, head_dim, G, k_new != nullptr, true);
         if (st.balanced != nullptr) ks.balanced = st.balanced;
         if (st.unit != nullptr) ks.unit = st.unit;
+        if (balanced && k_new != nullptr && st.balanced == nullptr) {
+            const Kernels plain = pick_tuned(dtype, head_dim, G, false, true);
+            if (plain.balanced != nullptr) {
+                ks.balanced = plain.balanced;
+                append_first = true;
+            }
+        }
     }
 
     DecodeArgs a;
@@ -616,6 +636,7 @@ int paged_decode_impl(const char* fn, void* out, const void* q, const void* k_ne
         a.S_max = 0;
         a.pps_auto = 0;
         a.fixed_S = 0;
+        if (append_first) launch_append(num_kv_heads, num_seqs, dtype, st, a);
         ks.balanced<<<dim3(a.nwg), 64 * kDecodeWaves, 0, st>>>(a);
         if (int e = check_launch(fn)) return e;
     } else {
@@ -638,11 +659,7 @@ int paged_decode_impl(const char* fn, void* out, const void* q, const void* k_ne
                 ks.split<<<grid, 64 * kDecodeWaves, 0, st>>>(a);
         } else {
             if (k_new != nullptr) {   // append first, then the plain generic decode
-                dim3 agrid(num_kv_heads, num_seqs);
-                if (dtype == LLKV_DTYPE_F32) append_new_rows_kernel<float><<<agrid, 64, 0, st>>>(a);
-                else if (dtype == LLKV_DTYPE_F16) append_new_rows_kernel<_Float16><<<agrid, 64, 0, st>>>(a);
-                else append_new_rows_kernel<bf16_t><<<agrid, 64, 0, st>>>(a);
-                a.knew = a.vnew = nullptr;
+                launch_append(num_kv_heads, num_seqs, dtype, st, a);
             }
             dim3 grid(p.S_max, num_q_heads, num_seqs);
             if (dtype == LLKV_DTYPE_F32) decode_generic_kernel<float><<<grid, 64, 0, st>>>(a);
