@@ -2,7 +2,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <climits>
 #include <cmath>
 #include <type_traits>
 #include <utility>
@@ -407,7 +406,7 @@ struct Smem {
             alignas(16) uint16_t k[2][BN * KPAD];
             alignas(16) uint16_t v[2][BN * KPAD];
         };
-        int order[6 * kRankUnits];   // prologue only: unit tiles, unit at each rank, q0, P, L, K/V offset
+        int order[6 * kRankUnits];   // prologue only: unit tiles, ranking keys, q0, P, L, K/V offset
     };
     int pages[kPageWindow];   // page ids [tbase, tbase + kPageWindow) of the sequence
 };
@@ -886,7 +885,8 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
     constexpr int DT = D / 16;              // 16-dim tiles of the output
     constexpr int KCH_T = BN * D / 4 / 256;          // 16-byte K chunks per thread
     constexpr int VT_N = (BN / 4) * (D / 4);           // V tasks (4 keys x 4 dims) per tile
-    constexpr int VT_T = (VT_N + 255) / 256;           // per thread
+    constexpr int VT_T = VT_N / 256;                   // per thread
+    static_assert(VT_N % 256 == 0, "V tasks spread evenly over the threads");
     __shared__ S sm;
 
     const int tid = threadIdx.x;
@@ -956,7 +956,7 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
     }
 #pragma unroll
     for (int j = 0; j < VT_T; ++j) {
-        const int task = (VT_N % 256 == 0 || tid + 256 * j < VT_N) ? tid + 256 * j : 0;   // idle: task 0's rows
+        const int task = tid + 256 * j;
         const int kq = task % (BN / 4), c = task / (BN / 4);   // keys 4kq .. 4kq+3, dims 4c .. 4c+3
         vslot[j] = CG ? 4 * kq : (4 * kq) >> 4;
         voff[j] = (CG ? 0u : (uint32_t)((4 * kq) & 15) * row_bytes) + (uint32_t)c * 16u;
@@ -1009,7 +1009,6 @@ void prefill_f32_kernel(MfmaPrefillArgs a) {
 #pragma unroll
         for (int j = 0; j < VT_T; ++j) {
             const int task = tid + 256 * j;
-            if (VT_N % 256 != 0 && task >= VT_N) break;
             const int kq = task % (BN / 4), c = task / (BN / 4);
 #pragma unroll
             for (int e = 0; e < 4; ++e)   // 4x4 transpose: V^T row 4c + e, keys 4kq .. 4kq+3
@@ -1914,10 +1913,8 @@ PrefillFn merge_kernel(int dtype, int head_dim) {
     return merge_for<bf16_t>(head_dim);
 }
 
-// Workspace: a header, then max_parts partial slots (Hq x BQ rows each), then one
-// slot for the merge kernel's table.
-constexpr size_t kPlanHeaderBytes = 256;
-
+// Workspace: max_parts partial slots (Hq x BQ rows each), then one slot for the
+// merge kernel's table.
 struct ChunkPlan {
     int qblocks, units;   // query blocks per sequence; bound of the units with rows
     int extra, parts;     // items beyond `units`; partial slots (0: nothing is cut)
@@ -1966,7 +1963,7 @@ size_t prefill_mfma_workspace(int N, int Hq, int head_dim, int block_size, int d
                               int max_q_len, int max_seq_len) {
     if (!prefill_mfma_handles(head_dim, block_size, dtype) || N <= 0 || total_q <= 0) return 0;
     const ChunkPlan c = chunk_plan(N, Hq, total_q, max_q_len, max_seq_len);
-    return c.parts > 0 ? kPlanHeaderBytes + (size_t)(c.parts + 1) * part_bytes(Hq, head_dim) : 0;
+    return c.parts > 0 ? (size_t)(c.parts + 1) * part_bytes(Hq, head_dim) : 0;
 }
 
 int launch_prefill_mfma(MfmaPrefillArgs a, int head_dim, int block_size, int dtype,
@@ -1994,7 +1991,7 @@ int launch_prefill_mfma(MfmaPrefillArgs a, int head_dim, int block_size, int dty
         workspace_bytes >= need) {
         a.max_parts = c.parts;
         a.extra_items = c.extra;
-        char* base = reinterpret_cast<char*>(workspace) + kPlanHeaderBytes;
+        char* base = reinterpret_cast<char*>(workspace);
         const size_t rows = (size_t)c.parts * a.Hq * BQ;
         a.part_lse = reinterpret_cast<float*>(base);
         a.part_o = a.part_lse + rows;
