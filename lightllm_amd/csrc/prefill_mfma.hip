@@ -1913,8 +1913,11 @@ PrefillFn merge_kernel(int dtype, int head_dim) {
     return merge_for<bf16_t>(head_dim);
 }
 
-// Workspace: max_parts partial slots (Hq x BQ rows each), then one slot for the
-// merge kernel's table.
+// Workspace: a 256-byte header (unused, part of the size that callers know), then
+// max_parts partial slots (Hq x BQ rows each), then one slot for the merge kernel's
+// table.
+constexpr size_t kHeaderBytes = 256;
+
 struct ChunkPlan {
     int qblocks, units;   // query blocks per sequence; bound of the units with rows
     int extra, parts;     // items beyond `units`; partial slots (0: nothing is cut)
@@ -1963,7 +1966,7 @@ size_t prefill_mfma_workspace(int N, int Hq, int head_dim, int block_size, int d
                               int max_q_len, int max_seq_len) {
     if (!prefill_mfma_handles(head_dim, block_size, dtype) || N <= 0 || total_q <= 0) return 0;
     const ChunkPlan c = chunk_plan(N, Hq, total_q, max_q_len, max_seq_len);
-    return c.parts > 0 ? (size_t)(c.parts + 1) * part_bytes(Hq, head_dim) : 0;
+    return c.parts > 0 ? kHeaderBytes + (size_t)(c.parts + 1) * part_bytes(Hq, head_dim) : 0;
 }
 
 int launch_prefill_mfma(MfmaPrefillArgs a, int head_dim, int block_size, int dtype,
@@ -1991,7 +1994,7 @@ int launch_prefill_mfma(MfmaPrefillArgs a, int head_dim, int block_size, int dty
         workspace_bytes >= need) {
         a.max_parts = c.parts;
         a.extra_items = c.extra;
-        char* base = reinterpret_cast<char*>(workspace);
+        char* base = reinterpret_cast<char*>(workspace) + kHeaderBytes;
         const size_t rows = (size_t)c.parts * a.Hq * BQ;
         a.part_lse = reinterpret_cast<float*>(base);
         a.part_o = a.part_lse + rows;
