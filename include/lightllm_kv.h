@@ -221,7 +221,9 @@ int llkv_paged_decode_noalloc(void* out, const void* q, const void* k_pool,
                               float scale, int dtype, void* stream);
 
 /* Fused KV append + paged decode: llkv_append of the step's new rows followed
- * by llkv_paged_decode, in one launch (plus the merge).  Replaces a
+ * by llkv_paged_decode, in one launch (plus the merge; the generic kernels, and
+ * large batches at head_dim 128 in 16 bits, append in a launch of their own).
+ * Replaces a
  * paged_attention call (src/engine/engine_server.cpp:1812-1817) together with
  * the per-sequence write_decode_kv loop (:1822-1854, two cudaMemcpy each); the
  * order is append first, so the new token attends to itself (the order of a
@@ -230,8 +232,8 @@ int llkv_paged_decode_noalloc(void* out, const void* q, const void* k_pool,
  * the new token: sequence b's new row goes to position seq_lens[b] - 1
  * (table page (L-1)/bs, row (L-1)%bs; skipped when that table entry is -1)
  * and attention covers positions [0, seq_lens[b]).  Results equal those of
- * the two calls made in order; the work-group that owns the new token reads
- * it from k_new / v_new while storing it to the pools.  Other arguments as
+ * the two calls made in order; in one launch, the work-group that owns the new
+ * token reads it from k_new / v_new while storing it to the pools.  Other arguments as
  * llkv_paged_decode. */
 int llkv_paged_decode_append(void* out, const void* q, const void* k_new,
                              const void* v_new, void* k_pool, void* v_pool,

@@ -273,7 +273,7 @@ __global__ __launch_bounds__(1024) void decode_merge_balanced_kernel(DecodeArgs 
 // 16 bits at 96 (252 -> 256), the 16-wave splits at 128 (116 -> 127) and in fp32 (70.5
 // -> 74.8).
 // The fused append at head_dim 128 in 16 bits has no registers for two forms of its
-// page loop (20 spilled).  Beyond this bound its rows are appended by a kernel of
+// page loop (8 .. 10 spilled).  Beyond this bound its rows are appended by a kernel of
 // their own and the plain call's kernels decode: 256 lognormal contexts of 32/8/128
 // fp16 389 -> 358 us, 128 x 50 .. 200 tokens under a bound of 16384 33 -> 31.
 constexpr int64_t kStreamBytes = 192ll << 20;

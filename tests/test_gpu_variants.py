@@ -440,6 +440,34 @@ def test_decode_shared_prefix_stays_cached():
     assert best[1] <= 1.12 * best[0], best
 
 
+def test_decode_streaming_choice_under_capture():
+    """A captured fused append + decode under a bound beyond the streaming rule follows the lengths of
+    each replay: beyond 192 MB, far below, and beyond again, with eager work between."""
+    B, hq, hkv, d, long = 40, 32, 8, 128, 1700
+    nb = B * ((long + 15) // 16)
+    pools = [torch.randn(nb, 16, hkv, d, device=DEV).half() for _ in range(2)]
+    q, kn, vn = (torch.randn(B, h, d, device=DEV).half() for h in (hq, hkv, hkv))
+    table = torch.randperm(nb, device=DEV).to(torch.int32).reshape(B, -1)
+    lens = torch.full((B,), long, dtype=torch.int32, device=DEV)
+    assert B * long * hkv * d * 4 > 192 << 20 and kc.decode_schedule(B, hq, hkv, d, long, q.dtype)[0] == "balanced"
+    ws = torch.empty(kc.decode_workspace_bytes(B, hq, hkv, d, 16, long), dtype=torch.uint8, device=DEV)
+    out = torch.empty_like(q)
+    step = lambda o, p: kc.paged_decode_append(q, kn, vn, *p, table, lens, long, out=o, workspace=ws)
+    step(out, pools)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(out, pools)
+    for n in (long, 33, long - 5):
+        lens.fill_(n)
+        eager = [p.clone() for p in pools]
+        want = step(torch.empty_like(q), eager)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and all(torch.equal(a, b) for a, b in zip(pools, eager)), n
+
+
 @pytest.mark.parametrize("extra", [0, 5])
 def test_gather_streaming_edge(extra):
     """Gathers on both sides of the streaming rule (4 x rows x row bytes at 288 MB), bit for bit."""
